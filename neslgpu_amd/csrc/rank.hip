@@ -21,6 +21,9 @@
 // indices).  The last pass leaves the sorted order of indices; the rank is
 // its inverse, rank[order[p]] = p (minus the segment offset), computed by
 // the coalesced permutation engine of partition.hip.
+//
+// A vector of at most kBlockRankMax keys is ranked by one workgroup in one
+// launch (k_rank_block).
 #include "cvl_hip.hpp"
 #include "segd.hpp"
 #include "lookback.hpp"
@@ -224,6 +227,190 @@ __global__ void k_hist_scan(unsigned *hist, unsigned *starts) {
         __syncthreads();
     }
     starts[p * kRadix + d] = sh[d] - v;
+}
+
+// ---------------------------------------------------------------- multisplit
+// A wave ranks its ITEMS x 64 keys by one 8-bit digit, stably: item j of a
+// lane is element j * 64 + lane of the wave's span, of which `count` exist.
+// dig: each item's digit; loc: its place among the wave's items of that
+// digit; cnt (256 counters of this wave, zero on entry): items per digit.
+// FULL: every element of the span exists (all but the last wave of a
+// vector), so no lane is masked out.
+template <bool FULL, int ITEMS, class KeyT>
+__device__ __forceinline__ void multisplit(const KeyT (&key)[ITEMS], int shift, int lane, int64_t count, unsigned *cnt,
+                                           unsigned (&dig)[ITEMS], unsigned (&loc)[ITEMS]) {
+#pragma unroll
+    for (int j = 0; j < ITEMS; j++) {
+        const bool in = FULL || (int64_t)j * kWave + lane < count;
+        const KeyT k = key[j];
+        const unsigned d = in ? (unsigned)((k >> shift) & 255) : 0u;
+        dig[j] = d;
+        // lanes of this round holding the same digit: those that agree
+        // with this lane in every bit of the digit, the AND over the
+        // bits of (lanes with the bit set) XNOR (all lanes if this lane
+        // has it set, none if not).  Per bit four instructions: the
+        // sign-extended bit, its lane mask (a compare of that value,
+        // which the compiler would otherwise rebuild from a shift of the
+        // digit), and one 3-input bit operation (v_bitop3, gfx950) per
+        // half of the mask: acc & ~(spread ^ mask), truth table 0x84
+        // over (spread, acc, mask).
+        uint32_t plo = ~0u, phi = ~0u;
+#pragma unroll
+        for (int b = 0; b < 8; b++) {
+            const uint32_t spread = (uint32_t)__builtin_amdgcn_sbfe((int)d, b, 1);   // 0 or ~0: bit b
+            const uint64_t bb = __builtin_amdgcn_uicmp(spread, 0u, 33);            // lanes with bit b (ICMP_NE)
+            plo = __builtin_amdgcn_bitop3_b32(spread, plo, (uint32_t)bb, 0x84);
+            phi = __builtin_amdgcn_bitop3_b32(spread, phi, (uint32_t)(bb >> 32), 0x84);
+        }
+        if constexpr (!FULL) {             // lanes past the end are no one's peers
+            const uint64_t act = ballot(in);
+            plo &= (uint32_t)act;
+            phi &= (uint32_t)(act >> 32);
+        }
+        // peers in lanes below this one (v_mbcnt: the set bits of a
+        // 64-lane mask below the current lane)
+        const unsigned before = __builtin_amdgcn_mbcnt_hi(phi, __builtin_amdgcn_mbcnt_lo(plo, 0u));
+        const uint64_t peers = ((uint64_t)phi << 32) | plo;
+        const unsigned old = cnt[d];
+        loc[j] = old + before;
+        // the highest lane of each digit group advances the counter
+        const bool leader = in && (peers >> lane) == 1ull;
+        if (leader) cnt[d] = old + before + 1;
+    }
+}
+
+// ---------------------------------------------------------------- short vectors
+// The rank of a vector that one workgroup holds: keys and original indices
+// (16 bits) stay in registers and LDS through all digit passes, so the call
+// is one launch with no host wait instead of 14 launches and one wait.  The
+// passes are bound by the multisplit's instructions on one CU (about 45 per
+// 64 keys and pass), the rest by barriers and LDS latency.  Against the
+// passes below, us per call: 1000 ints 67 -> 7.4, 5000 74 -> 16, 16000 99 ->
+// 37; 1000 doubles 126 -> 14, 8192 146 -> 43.
+// ITEMS: keys per lane, the fewest that hold the vector (idle lanes still
+// take their share of every round).
+constexpr int kBlockRankThreads = 1024;
+
+template <class KeyT, int ITEMS>
+__global__ __launch_bounds__(kBlockRankThreads) void k_rank_block(const void *__restrict__ s, int n, int up,
+                                                                  int *__restrict__ rank) {
+    constexpr int W = kBlockRankThreads / kWave, TILE = kBlockRankThreads * ITEMS, SPAN = kWave * ITEMS;
+    constexpr int NW = sizeof(KeyT) / 4, P = sizeof(KeyT);
+    static_assert(TILE <= 65536, "16-bit indices");
+    __shared__ __attribute__((aligned(16))) unsigned s_cnt[W][kRadix];
+    __shared__ KeyT s_key[TILE];
+    __shared__ unsigned short s_idx[TILE];
+    __shared__ uint32_t s_or[NW][W];
+    const int tid = threadIdx.x, w = tid / kWave, lane = tid % kWave;
+    const int wb = w * SPAN;
+    auto key_at = [&](int e) -> KeyT {
+        if constexpr (NW == 2) return dbl_key(((const double *)s)[e], up);
+        else return int_key(((const int *)s)[e], up);
+    };
+    auto clear = [&] {
+        const u32x4 z = {0u, 0u, 0u, 0u};
+        for (int i = tid; i < W * kRadix / 4; i += kBlockRankThreads) ((u32x4 *)&s_cnt[0][0])[i] = z;
+    };
+    KeyT key[ITEMS];
+    unsigned idx[ITEMS];
+    const KeyT k0 = key_at(0);
+    KeyT x = 0;
+#pragma unroll
+    for (int j = 0; j < ITEMS; j++) {
+        const int e = wb + j * kWave + lane;
+        idx[j] = (unsigned)e;
+        key[j] = e < n ? key_at(e) : k0;
+    }
+    clear();
+#pragma unroll
+    for (int j = 0; j < ITEMS; j++) x |= key[j] ^ k0;
+#pragma unroll
+    for (int k = 0; k < NW; k++) {
+        const uint32_t r = wave_reduce((uint32_t)((uint64_t)x >> (32 * k)), OrU());
+        if (lane == 0) s_or[k][w] = r;
+    }
+    __syncthreads();
+    // the bits in which some key differs from key 0: a pass none of whose
+    // bits is among them keeps the order and is skipped
+    uint64_t diff = 0;
+#pragma unroll
+    for (int k = 0; k < NW; k++) {
+        uint32_t r = 0;
+#pragma unroll
+        for (int i = 0; i < W; i++) r |= s_or[k][i];
+        diff |= (uint64_t)r << (32 * k);
+    }
+    if (diff == 0) {                       // all keys equal
+        for (int i = tid; i < n; i += kBlockRankThreads) rank[i] = i;
+        return;
+    }
+    for (int p = 0; p < P; p++) {
+        const uint64_t rest = diff >> (8 * p);
+        if (rest == 0) break;
+        if ((rest & 255) == 0) continue;
+        const bool last = (rest >> 8) == 0;
+        unsigned dig[ITEMS], loc[ITEMS];
+        if (wb + SPAN <= n) multisplit<true>(key, 8 * p, lane, SPAN, s_cnt[w], dig, loc);
+        else if (wb < n) multisplit<false>(key, 8 * p, lane, n - wb, s_cnt[w], dig, loc);
+        __syncthreads();
+        if (w == 0) {
+            // where each wave's items of each digit start: lane l takes the
+            // digits 4l .. 4l+3
+            u32x4 t = {0u, 0u, 0u, 0u};
+#pragma unroll 4
+            for (int i = 0; i < W; i++) t += *(const u32x4 *)&s_cnt[i][4 * lane];
+            const unsigned all = t.x + t.y + t.z + t.w;
+            const unsigned at = wave_inclusive_scan(all, AddU()) - all;
+            u32x4 run = {at, at + t.x, at + t.x + t.y, at + t.x + t.y + t.z};
+#pragma unroll 4
+            for (int i = 0; i < W; i++) {
+                const u32x4 c = *(const u32x4 *)&s_cnt[i][4 * lane];
+                *(u32x4 *)&s_cnt[i][4 * lane] = run;
+                run += c;
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < ITEMS; j++) {
+            if (wb + j * kWave + lane >= n) continue;
+            const unsigned at = s_cnt[w][(key[j] >> (8 * p)) & 255] + loc[j];
+            if (last) {
+                s_idx[idx[j]] = (unsigned short)at;      // the rank, by original index
+            } else {
+                s_key[at] = key[j];
+                s_idx[at] = (unsigned short)idx[j];
+            }
+        }
+        __syncthreads();
+        if (last) break;
+        clear();
+#pragma unroll
+        for (int j = 0; j < ITEMS; j++) {
+            const int e = wb + j * kWave + lane;
+            if (e < n) {
+                key[j] = s_key[e];
+                idx[j] = s_idx[e];
+            }
+        }
+        __syncthreads();
+    }
+    for (int i = tid; i < n; i += kBlockRankThreads) rank[i] = (int)s_idx[i];
+}
+
+// The longest vector it takes: 112 KiB of the 160 KiB LDS for ints, 96 KiB
+// for doubles.  There it still takes less than half the time of the passes
+// (figures above); twice as many keys do not fit.
+constexpr int kBlockRankMax4 = 16 * kBlockRankThreads, kBlockRankMax8 = 8 * kBlockRankThreads;
+
+template <class KeyT, int ITEMS>
+static void launch_rank_block(const void *s, int n, bool up, int *rank) {
+    if constexpr (ITEMS > 1)
+        if (n <= (ITEMS > 8 ? ITEMS - 4 : ITEMS > 4 ? ITEMS - 2 : ITEMS - 1) * kBlockRankThreads) {
+            launch_rank_block<KeyT, (ITEMS > 8 ? ITEMS - 4 : ITEMS > 4 ? ITEMS - 2 : ITEMS - 1)>(s, n, up, rank);
+            return;
+        }
+    k_rank_block<KeyT, ITEMS><<<1, kBlockRankThreads, 0, g_stream>>>(s, n, up, rank);
+    LAUNCHCHECK();
 }
 
 // ---------------------------------------------------------------- one pass
@@ -502,51 +689,8 @@ __global__ __launch_bounds__(kRankThreads) void k_rank_pass(PassArgs a) {
         idx[j] = ix;
     }
 loaded:
-    // FULL: every element of the wave's span exists (all but the last
-    // wave of the vector), so no lane is masked out.
-    auto multisplit = [&](auto full) {
-        constexpr bool FULL = decltype(full)::value;
-#pragma unroll
-        for (int j = 0; j < kRankItems; j++) {
-            const bool in = FULL || wb + (int64_t)j * kWave + lane < a.n;
-            const KeyT k = key[j];
-            const unsigned d = in ? (unsigned)((k >> a.shift) & 255) : 0u;
-            dig[j] = d;
-            // lanes of this round holding the same digit: those that agree
-            // with this lane in every bit of the digit, the AND over the
-            // bits of (lanes with the bit set) XNOR (all lanes if this lane
-            // has it set, none if not).  Per bit four instructions: the
-            // sign-extended bit, its lane mask (a compare of that value,
-            // which the compiler would otherwise rebuild from a shift of the
-            // digit), and one 3-input bit operation (v_bitop3, gfx950) per
-            // half of the mask: acc & ~(spread ^ mask), truth table 0x84
-            // over (spread, acc, mask).
-            uint32_t plo = ~0u, phi = ~0u;
-#pragma unroll
-            for (int b = 0; b < 8; b++) {
-                const uint32_t spread = (uint32_t)__builtin_amdgcn_sbfe((int)d, b, 1);   // 0 or ~0: bit b
-                const uint64_t bb = __builtin_amdgcn_uicmp(spread, 0u, 33);            // lanes with bit b (ICMP_NE)
-                plo = __builtin_amdgcn_bitop3_b32(spread, plo, (uint32_t)bb, 0x84);
-                phi = __builtin_amdgcn_bitop3_b32(spread, phi, (uint32_t)(bb >> 32), 0x84);
-            }
-            if constexpr (!FULL) {             // lanes past the end are no one's peers
-                const uint64_t act = ballot(in);
-                plo &= (uint32_t)act;
-                phi &= (uint32_t)(act >> 32);
-            }
-            // peers in lanes below this one (v_mbcnt: the set bits of a
-            // 64-lane mask below the current lane)
-            const unsigned before = __builtin_amdgcn_mbcnt_hi(phi, __builtin_amdgcn_mbcnt_lo(plo, 0u));
-            const uint64_t peers = ((uint64_t)phi << 32) | plo;
-            const unsigned old = s_cnt[w][d];
-            loc[j] = old + before;
-            // the highest lane of each digit group advances the counter
-            const bool leader = in && (peers >> lane) == 1ull;
-            if (leader) s_cnt[w][d] = old + before + 1;
-        }
-    };
-    if (wb + kWaveSpan <= a.n) multisplit(std::true_type{});
-    else multisplit(std::false_type{});
+    if (wb + kWaveSpan <= a.n) multisplit<true>(key, a.shift, lane, kWaveSpan, s_cnt[w], dig, loc);
+    else multisplit<false>(key, a.shift, lane, a.n - wb, s_cnt[w], dig, loc);
     __syncthreads();
 
     // Per digit: wave starts within the digit, the tile count, and the
@@ -737,6 +881,11 @@ void rank_run(int *rank, const void *s, int64_t n, bool dbl, bool up, const void
     unsigned *tile_ofs = (unsigned *)(b + L.status);
     uint64_t *scan_status = (uint64_t *)(b + L.scan_status);
     const bool segmented = sd != nullptr && m > 1;
+    if (!segmented && n <= (dbl ? kBlockRankMax8 : kBlockRankMax4)) {
+        if (dbl) launch_rank_block<uint64_t, kBlockRankMax8 / kBlockRankThreads>(s, (int)n, up, rank);
+        else launch_rank_block<uint32_t, kBlockRankMax4 / kBlockRankThreads>(s, (int)n, up, rank);
+        return;
+    }
     SegdView seg(sd, n, segmented ? m : 0);
     const int key_passes = dbl ? 8 : 4;
     int seg_passes = 0;

@@ -22,8 +22,10 @@
 // its inverse, rank[order[p]] = p (minus the segment offset), computed by
 // the coalesced permutation engine of partition.hip.
 //
-// A vector of at most kBlockRankMax keys is ranked by one workgroup in one
-// launch (k_rank_block).
+// A vector of at most kBlockRankMax4 ints or kBlockRankMax8 doubles is ranked
+// by one workgroup in one launch (k_rank_block).  Up to kRankDirectMax keys
+// the passes run without the column scan (grouped tile counts) and the last
+// one stores the ranks itself (kDirect).
 #include "cvl_hip.hpp"
 #include "segd.hpp"
 #include "lookback.hpp"
@@ -52,7 +54,10 @@ constexpr int kRankThreads = CVLHIP_RANK_THREADS;        // waves of 64
 static_assert(kRankThreads >= 256, "one thread per digit");
 constexpr int kRankItems = CVLHIP_RANK_ITEMS;            // per lane
 constexpr int kRankTile = kRankThreads * kRankItems;     // keys per tile
-constexpr int kWaveSpan = kWave * kRankItems;            // consecutive keys per wave
+
+// Tiles of vectors short enough that 4096-key tiles would leave most CUs
+// without one.
+constexpr int kRankSmallThreads = 256, kRankSmallItems = 4;
 
 // ---------------------------------------------------------------- key transforms
 // KeyT: uint32_t (int ranks) or uint64_t (double ranks, low field in the low
@@ -445,7 +450,24 @@ struct PassArgs {
     uint2 *pairs;
     const unsigned *tile_ofs2;
     int clog;
+    // Grouped tiles: tile_ofs holds the tiles' own counts, groups the
+    // counts of each kRankGroup tiles together (ngroups x 256), and the pass
+    // adds up what lies before its tile itself; starts is not read.
+    unsigned *groups;
+    int64_t ngroups;
+    // The last pass with a direct inverse: rank[index] = position, minus the
+    // start of the index's segment when rel is set.
+    int *rank;
+    int rel;
 };
+
+constexpr int kRankGroup = 32;            // tiles per group
+constexpr int kRankGroups = 64;           // most groups that a pass adds up
+
+// Which order a pass leaves: kOrder writes the element order (and the keys
+// the next passes need), kFuse the inverse's first partition pass, kDirect
+// the ranks themselves.
+enum RankOut { kOrder, kFuse, kDirect };
 
 // Key of element e for this pass (ix = its original index).
 template <class KeyT>
@@ -492,8 +514,8 @@ __device__ __forceinline__ void store_key(const PassArgs &a, int64_t pos, KeyT k
 // With ORW (the first pass, launched before the host knows which passes
 // run) it also writes the bits in which the tile's keys differ from key 0
 // to or_parts[2 tile], [2 tile + 1] (low, high 32 bits) for k_or_post.
-template <class KeyT, bool B2, bool ORW = false>
-__global__ __launch_bounds__(kRankThreads) void k_rank_hist(PassArgs a, unsigned *__restrict__ hist,
+template <class KeyT, bool B2, bool ORW = false, int TH = kRankThreads, int IT = kRankItems>
+__global__ __launch_bounds__(TH) void k_rank_hist(PassArgs a, unsigned *__restrict__ hist,
                                                             unsigned *__restrict__ hist2,
                                                             uint32_t *__restrict__ or_parts = nullptr) {
     __shared__ unsigned s_hist[kRadix];
@@ -503,21 +525,21 @@ __global__ __launch_bounds__(kRankThreads) void k_rank_hist(PassArgs a, unsigned
     // (read first, so that its latency hides behind the tile's loads)
     KeyT k0 = 0;
     if constexpr (ORW) k0 = pass_key<KeyT>(a, 0, 0);
-    for (int i = tid; i < kRadix; i += kRankThreads) {
+    for (int i = tid; i < kRadix; i += TH) {
         s_hist[i] = 0;
         if constexpr (B2) s_hist2[i] = 0;
     }
     __syncthreads();
     const int64_t tile = blockIdx.x;      // rows are whole 1 KiB stores: launch order
-    const int64_t t0 = tile * kRankTile;
-    // Item j is element t0 + ((j / 4) * kRankThreads + tid) * 4 + j % 4: runs
+    const int64_t t0 = tile * (TH * IT);
+    // Item j is element t0 + ((j / 4) * TH + tid) * 4 + j % 4: runs
     // of four per lane, one 16-byte load each for 4-byte keys.
-    static_assert(kRankItems % 4 == 0, "runs of four keys per lane");
-    KeyT kv[kRankItems];
-    bool in[kRankItems];
+    static_assert(IT % 4 == 0, "runs of four keys per lane");
+    KeyT kv[IT];
+    bool in[IT];
 #pragma unroll
-    for (int g = 0; g < kRankItems / 4; g++) {
-        const int64_t e0 = t0 + ((int64_t)g * kRankThreads + tid) * 4;
+    for (int g = 0; g < IT / 4; g++) {
+        const int64_t e0 = t0 + ((int64_t)g * TH + tid) * 4;
         if (a.vec4 && e0 + 4 <= a.n) {
             const u32x4 w = load_fields4(a, e0);
             const uint32_t x[4] = {w.x, w.y, w.z, w.w};
@@ -538,17 +560,17 @@ __global__ __launch_bounds__(kRankThreads) void k_rank_hist(PassArgs a, unsigned
         }
     }
 #pragma unroll
-    for (int j = 0; j < kRankItems; j++)
+    for (int j = 0; j < IT; j++)
         if (in[j]) atomicAdd(&s_hist[(kv[j] >> a.shift) & 255], 1u);
     if constexpr (ORW) {
         // the bits in which some key of the tile differs from key 0 of the
         // vector (the same reference in every tile): a digit takes one value
         // over all keys iff none of its bits differs anywhere
         constexpr int NW = sizeof(KeyT) / 4;
-        __shared__ uint32_t s_or[kRankThreads / kWave][NW];
+        __shared__ uint32_t s_or[TH / kWave][NW];
         KeyT x = 0;
 #pragma unroll
-        for (int j = 0; j < kRankItems; j++)
+        for (int j = 0; j < IT; j++)
             if (in[j]) x |= kv[j] ^ k0;
         const int w = tid / kWave, lane = tid % kWave;
 #pragma unroll
@@ -561,15 +583,15 @@ __global__ __launch_bounds__(kRankThreads) void k_rank_hist(PassArgs a, unsigned
             uint32_t r = 0;
             if (tid < NW)
 #pragma unroll
-                for (int i = 0; i < kRankThreads / kWave; i++) r |= s_or[i][tid];
+                for (int i = 0; i < TH / kWave; i++) r |= s_or[i][tid];
             or_parts[2 * tile + tid] = r;
         }
     }
     if constexpr (B2) {
         // the elements' original indices: children of the inverse
 #pragma unroll
-        for (int g = 0; g < kRankItems / 4; g++) {
-            const int64_t e0 = t0 + ((int64_t)g * kRankThreads + tid) * 4;
+        for (int g = 0; g < IT / 4; g++) {
+            const int64_t e0 = t0 + ((int64_t)g * TH + tid) * 4;
             int ix[4];
             if (a.idx_in && e0 + 4 <= a.n) {
                 const u32x4 w = *(const u32x4 *)((const uint32_t *)a.idx_in + e0);
@@ -584,27 +606,31 @@ __global__ __launch_bounds__(kRankThreads) void k_rank_hist(PassArgs a, unsigned
         }
     }
     __syncthreads();
-    for (int d = tid; d < kRadix; d += kRankThreads) {
-        hist[tile * kRadix + d] = s_hist[d];
+    for (int d = tid; d < kRadix; d += TH) {
+        const unsigned c = s_hist[d];
+        hist[tile * kRadix + d] = c;
+        if (a.groups && c) atomicAdd(a.groups + (tile / kRankGroup) * kRadix + d, c);
         if constexpr (B2) hist2[tile * kRadix + d] = s_hist2[d];
     }
 }
 
 // KOUT: bytes per key written to keys_out (a.kout), 0 when no keys are.
-// FUSE (KOUT 0): the pass writes the inverse's first partition pass
-// (a.pairs) instead of the order.
-template <class KeyT, int KOUT, bool FUSE = false>
-__global__ __launch_bounds__(kRankThreads) void k_rank_pass(PassArgs a) {
-    static_assert(!FUSE || KOUT == 0, "the fused last pass writes no keys");
-    constexpr int W = kRankThreads / kWave;
+// OUT: what it leaves (RankOut); GRP: grouped tile counts; TH x IT: the tile.
+template <class KeyT, int KOUT, RankOut OUT, bool GRP, int TH = kRankThreads, int IT = kRankItems>
+__global__ __launch_bounds__(TH) void k_rank_pass(PassArgs a) {
+    static_assert(OUT == kOrder || KOUT == 0, "the last pass writes no keys");
+    static_assert(TH >= kRadix, "one thread per digit");
+    constexpr bool FUSE = OUT == kFuse;
+    constexpr int W = TH / kWave;
+    constexpr int kWaveSpan = kWave * IT;     // consecutive keys per wave
     // s_cnt: per-wave digit counts, then per-wave starts within a digit;
     // s_stage: keys, then (reinterpreted) indices, in digit order.  FUSE:
     // the 8-byte pairs in child order, staged once every position is known,
     // over both (then dead): 32 KiB instead of 8 + 32, so three workgroups
     // of LDS become four.
     constexpr int kCntBytes = W * kRadix * 4;
-    constexpr int kStageBytes = kRankTile * (int)sizeof(KeyT);
-    constexpr int kPairBytes = kRankTile * 8;
+    constexpr int kStageBytes = (TH * IT) * (int)sizeof(KeyT);
+    constexpr int kPairBytes = (TH * IT) * 8;
     constexpr int kRaw = (FUSE && kPairBytes > kCntBytes + kStageBytes) ? kPairBytes : kCntBytes + kStageBytes;
     __shared__ __attribute__((aligned(16))) unsigned char s_raw[kRaw];
     unsigned(*const s_cnt)[kRadix] = (unsigned(*)[kRadix])s_raw;
@@ -612,30 +638,56 @@ __global__ __launch_bounds__(kRankThreads) void k_rank_pass(PassArgs a) {
     __shared__ unsigned s_tot[kRadix];
     __shared__ unsigned s_lstart[kRadix];     // tile-local start of each digit's run
     __shared__ unsigned s_gbase[kRadix];      // global position of the run
-    __shared__ unsigned char s_dig[FUSE ? 1 : kRankTile];
+    __shared__ unsigned char s_dig[FUSE ? 1 : (TH * IT)];
     __shared__ unsigned s_c2[FUSE ? kRadix : 1];   // FUSE: per-child counts, then starts, of the tile
     __shared__ unsigned s_g2[FUSE ? kRadix : 1];   // FUSE: the tile's slot in each child
+    __shared__ unsigned s_all[GRP ? kRadix : 1];   // GRP: each digit's count in the whole vector
     __shared__ unsigned s_placed;                  // FUSE: pairs staged
     __shared__ unsigned s_tile;
 
     const int tid = threadIdx.x;
     const int w = tid / kWave, lane = tid % kWave;
-    for (int i = tid; i < W * kRadix; i += kRankThreads) (&s_cnt[0][0])[i] = 0;
+    for (int i = tid; i < W * kRadix; i += TH) (&s_cnt[0][0])[i] = 0;
     if constexpr (FUSE)
-        for (int i = tid; i < kRadix; i += kRankThreads) s_c2[i] = 0;
+        for (int i = tid; i < kRadix; i += TH) s_c2[i] = 0;
     // a chained pass numbers its tiles in the order they start; the
     // order of the tiles' runs within a digit is then their data order
     if (kRankChain && a.chain && tid == 0) s_tile = atomicAdd(a.ticket, 1u);
     __syncthreads();
     const int64_t tile = (kRankChain && a.chain) ? (int64_t)s_tile : xcd_tile(blockIdx.x, gridDim.x);
-    const int64_t t0 = tile * kRankTile;
-    const int64_t count = a.n - t0 < kRankTile ? a.n - t0 : kRankTile;
+    const int64_t t0 = tile * (TH * IT);
+    const int64_t count = a.n - t0 < (TH * IT) ? a.n - t0 : (TH * IT);
     const int64_t wb = t0 + (int64_t)w * kWaveSpan;
 
-    KeyT key[kRankItems];
-    int idx[kRankItems];
-    unsigned dig[kRankItems];
-    unsigned loc[kRankItems];
+    if constexpr (GRP) {
+        // Elements of each digit in the earlier tiles of this tile's group
+        // and in the earlier groups, and in all groups: at most kRankGroup +
+        // kRankGroups loads per thread, ahead of the tile's own loads.
+        const int64_t g = tile / kRankGroup;
+        for (int q = tid; q < 2 * kRadix; q += TH) {
+            const int d = q % kRadix;
+            unsigned before = 0, all = 0;
+            if (q < kRadix) {
+#pragma unroll 8
+                for (int64_t r = g * kRankGroup; r < tile; r++) before += a.tile_ofs[r * kRadix + d];
+                s_gbase[d] = before;
+            } else {
+#pragma unroll 8
+                for (int64_t r = 0; r < a.ngroups; r++) {
+                    const unsigned c = a.groups[r * kRadix + d];
+                    all += c;
+                    before += r < g ? c : 0u;
+                }
+                s_lstart[d] = before;
+                s_all[d] = all;
+            }
+        }
+    }
+
+    KeyT key[IT];
+    int idx[IT];
+    unsigned dig[IT];
+    unsigned loc[IT];
 
     // Item j of a lane is element wb + j*64 + lane: each round of the
     // multisplit below holds 64 consecutive elements, which keeps it stable.
@@ -644,11 +696,11 @@ __global__ __launch_bounds__(kRankThreads) void k_rank_pass(PassArgs a) {
     // wave's own part of s_stage, which is free until the staging phase.
     if constexpr (sizeof(KeyT) == 4) {
         if (a.vec4 && wb + kWaveSpan <= a.n) {
-            static_assert(kRankItems % 4 == 0, "runs of four keys per lane");
+            static_assert(IT % 4 == 0, "runs of four keys per lane");
             uint32_t *sw = (uint32_t *)s_stage + (int64_t)w * kWaveSpan;
-            auto transpose = [&](auto load4, uint32_t (&out)[kRankItems]) {
+            auto transpose = [&](auto load4, uint32_t (&out)[IT]) {
 #pragma unroll
-                for (int g = 0; g < kRankItems / 4; g++) {
+                for (int g = 0; g < IT / 4; g++) {
                     const u32x4 v = load4(wb + g * 4 * kWave + 4 * lane);
                     *(u32x4 *)(sw + g * 4 * kWave + 4 * lane) = v;
                 }
@@ -656,28 +708,28 @@ __global__ __launch_bounds__(kRankThreads) void k_rank_pass(PassArgs a) {
                 __builtin_amdgcn_wave_barrier();
                 __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
-                for (int j = 0; j < kRankItems; j++) out[j] = sw[j * kWave + lane];
+                for (int j = 0; j < IT; j++) out[j] = sw[j * kWave + lane];
                 __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
                 __builtin_amdgcn_wave_barrier();
                 __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
             };
-            uint32_t raw[kRankItems];
+            uint32_t raw[IT];
             transpose([&](int64_t e) { return load_fields4(a, e); }, raw);
 #pragma unroll
-            for (int j = 0; j < kRankItems; j++) key[j] = (KeyT)(a.source == 0 ? int_key((int)raw[j], a.up) : raw[j]);
+            for (int j = 0; j < IT; j++) key[j] = (KeyT)(a.source == 0 ? int_key((int)raw[j], a.up) : raw[j]);
             if (a.idx_in) {
                 transpose([&](int64_t e) { return *(const u32x4 *)((const uint32_t *)a.idx_in + e); }, raw);
 #pragma unroll
-                for (int j = 0; j < kRankItems; j++) idx[j] = (int)raw[j];
+                for (int j = 0; j < IT; j++) idx[j] = (int)raw[j];
             } else {
 #pragma unroll
-                for (int j = 0; j < kRankItems; j++) idx[j] = (int)(wb + (int64_t)j * kWave + lane);
+                for (int j = 0; j < IT; j++) idx[j] = (int)(wb + (int64_t)j * kWave + lane);
             }
             goto loaded;
         }
     }
 #pragma unroll
-    for (int j = 0; j < kRankItems; j++) {
+    for (int j = 0; j < IT; j++) {
         const int64_t e = wb + (int64_t)j * kWave + lane;
         KeyT k = 0;
         int ix = 0;
@@ -705,10 +757,14 @@ loaded:
             run += c;
         }
         s_tot[d] = run;
-        const unsigned prefix = (kRankChain && a.chain)
-                                    ? chain_exclusive(a.chain, tile, kRadix, d, run, a.parity, a.err)
-                                    : a.tile_ofs[tile * kRadix + d];
-        s_gbase[d] = a.starts[d] + prefix;
+        if constexpr (GRP) {
+            s_gbase[d] += s_lstart[d];
+        } else {
+            const unsigned prefix = (kRankChain && a.chain)
+                                        ? chain_exclusive(a.chain, tile, kRadix, d, run, a.parity, a.err)
+                                        : a.tile_ofs[tile * kRadix + d];
+            s_gbase[d] = a.starts[d] + prefix;
+        }
     }
     __syncthreads();
     // tile-local digit starts: exclusive scan of the 256 totals (one wave)
@@ -717,15 +773,40 @@ loaded:
 #pragma unroll
         for (int i = 0; i < kRadix / kWave; i++) { c[i] = s_tot[tid * (kRadix / kWave) + i]; t += c[i]; }
         unsigned run = wave_inclusive_scan(t, AddU()) - t;
+        unsigned gc[kRadix / kWave] = {}, grun = 0;     // grouped: the digits' starts in the whole vector
+        if constexpr (GRP) {
+            unsigned gt = 0;
+#pragma unroll
+            for (int i = 0; i < kRadix / kWave; i++) { gc[i] = s_all[tid * (kRadix / kWave) + i]; gt += gc[i]; }
+            grun = wave_inclusive_scan(gt, AddU()) - gt;
+        }
 #pragma unroll
         for (int i = 0; i < kRadix / kWave; i++) {
             const int d = tid * (kRadix / kWave) + i;
             s_lstart[d] = run;
-            s_gbase[d] -= run;       // now: global position of local slot 0 of digit d's run
+            s_gbase[d] += grun - run;       // now: global position of local slot 0 of digit d's run
             run += c[i];
+            grun += gc[i];
         }
     }
     __syncthreads();
+
+    if constexpr (OUT == kDirect) {
+        // Every element's sorted position is its rank: store it where the
+        // element came from.
+#pragma unroll
+        for (int j = 0; j < IT; j++) {
+            const int64_t e = wb + (int64_t)j * kWave + lane;
+            if (e >= a.n) continue;
+            const unsigned d = dig[j];
+            const unsigned pos = s_gbase[d] + s_lstart[d] + s_cnt[w][d] + loc[j];
+            if ((unsigned)idx[j] < (unsigned)a.n)
+                a.rank[idx[j]] = (int)pos - (a.rel ? a.seg.offs[a.seg.seg_of(idx[j])] : 0);
+            else
+                atomicOr(a.err, 1u);
+        }
+        return;
+    }
 
     if constexpr (FUSE) {
         // Every element's sorted position is known here: place the pair
@@ -733,9 +814,9 @@ loaded:
         // partition pass, staged in child order, each child's run written
         // contiguously at the tile's slot in that child.
         uint2 *const s_pair = (uint2 *)s_raw;   // written only after the barrier below: s_cnt is read here
-        unsigned ch[kRankItems], rk[kRankItems], pos[kRankItems];
+        unsigned ch[IT], rk[IT], pos[IT];
 #pragma unroll
-        for (int j = 0; j < kRankItems; j++) {
+        for (int j = 0; j < IT; j++) {
             const int64_t e = wb + (int64_t)j * kWave + lane;
             ch[j] = 0xFFFFFFFFu;
             if (e < a.n) {
@@ -762,17 +843,17 @@ loaded:
             }
             if (tid == kWave - 1) s_placed = run;
         }
-        for (int i = tid; i < kRadix; i += kRankThreads) s_g2[i] = a.tile_ofs2[tile * kRadix + i];
+        for (int i = tid; i < kRadix; i += TH) s_g2[i] = a.tile_ofs2[tile * kRadix + i];
         __syncthreads();
 #pragma unroll
-        for (int j = 0; j < kRankItems; j++)
+        for (int j = 0; j < IT; j++)
             if (ch[j] != 0xFFFFFFFFu) s_pair[s_c2[ch[j]] + rk[j]] = make_uint2((unsigned)idx[j], pos[j]);
         __syncthreads();
         // s_pair[0 .. placed): the tile's elements with a valid index, by
         // child (index < n < 2^(clog + 8), so every child is below 256)
         const int placed = (int)s_placed;
         const int64_t csize = (int64_t)1 << a.clog;
-        for (int i = tid; i < placed; i += kRankThreads) {
+        for (int i = tid; i < placed; i += TH) {
             const uint2 pr = s_pair[i];
             const unsigned c = pr.x >> a.clog;
             const int64_t at = (int64_t)c * csize + s_g2[c] + (i - s_c2[c]);
@@ -785,9 +866,9 @@ loaded:
 
     // Stage in digit order, then write each digit's run contiguously:
     // first the keys (when a later pass needs them), then the indices.
-    unsigned slot[kRankItems];
+    unsigned slot[IT];
 #pragma unroll
-    for (int j = 0; j < kRankItems; j++) {
+    for (int j = 0; j < IT; j++) {
         const int64_t e = wb + (int64_t)j * kWave + lane;
         slot[j] = 0;
         if (e < a.n) {
@@ -797,19 +878,19 @@ loaded:
         }
     }
     __syncthreads();
-    // Staged element i = tid + k * kRankThreads goes to s_gbase[its digit]
+    // Staged element i = tid + k * TH goes to s_gbase[its digit]
     // + i, for the keys and then for the indices.  (s_gbase[d] >= 0: the
     // tile's elements below digit d are among all elements below it.)
-    unsigned spos[kRankItems];
+    unsigned spos[IT];
 #pragma unroll
-    for (int k = 0; k < kRankItems; k++) {
-        const int i = tid + k * kRankThreads;
+    for (int k = 0; k < IT; k++) {
+        const int i = tid + k * TH;
         spos[k] = i < count ? s_gbase[s_dig[i]] + (unsigned)i : 0xFFFFFFFFu;
     }
     if constexpr (KOUT > 0) {
 #pragma unroll
-        for (int k = 0; k < kRankItems; k++) {
-            const int i = tid + k * kRankThreads;
+        for (int k = 0; k < IT; k++) {
+            const int i = tid + k * TH;
             if (i < count) {
                 if (spos[k] < a.n) store_key<KeyT, KOUT>(a, spos[k], s_stage[i]);
                 else atomicOr(a.err, 1u);
@@ -819,14 +900,14 @@ loaded:
     }
     int *s_idx = (int *)s_stage;
 #pragma unroll
-    for (int j = 0; j < kRankItems; j++) {
+    for (int j = 0; j < IT; j++) {
         const int64_t e = wb + (int64_t)j * kWave + lane;
         if (e < a.n) s_idx[slot[j]] = idx[j];
     }
     __syncthreads();
 #pragma unroll
-    for (int k = 0; k < kRankItems; k++) {
-        const int i = tid + k * kRankThreads;
+    for (int k = 0; k < IT; k++) {
+        const int i = tid + k * TH;
         if (i < count) {
             if (spos[k] < a.n) a.idx_out[spos[k]] = s_idx[i];
             else atomicOr(a.err, 1u);
@@ -870,6 +951,55 @@ struct RankScratch {
 
 static unsigned *g_hist_host = nullptr;
 
+template <int TH, int IT, bool B2, bool ORW>
+static void launch_hist(const PassArgs &a, int64_t tiles, bool dbl, unsigned *hist, unsigned *hist2, uint32_t *or_parts) {
+    if (dbl) k_rank_hist<uint64_t, B2, ORW, TH, IT><<<(unsigned)tiles, TH, 0, g_stream>>>(a, hist, hist2, or_parts);
+    else k_rank_hist<uint32_t, B2, ORW, TH, IT><<<(unsigned)tiles, TH, 0, g_stream>>>(a, hist, hist2, or_parts);
+    LAUNCHCHECK();
+}
+
+// An order-writing pass: the kernel of the key width it writes.
+template <bool GRP, int TH, int IT>
+static void launch_order(const PassArgs &a, dim3 grid, bool dbl) {
+    if (dbl) {
+        if (a.keys_out) k_rank_pass<uint64_t, 8, kOrder, GRP, TH, IT><<<grid, TH, 0, g_stream>>>(a);
+        else k_rank_pass<uint64_t, 0, kOrder, GRP, TH, IT><<<grid, TH, 0, g_stream>>>(a);
+    } else if (!a.keys_out) {
+        k_rank_pass<uint32_t, 0, kOrder, GRP, TH, IT><<<grid, TH, 0, g_stream>>>(a);
+    } else if (a.kout == 1) {
+        k_rank_pass<uint32_t, 1, kOrder, GRP, TH, IT><<<grid, TH, 0, g_stream>>>(a);
+    } else if (a.kout == 2) {
+        k_rank_pass<uint32_t, 2, kOrder, GRP, TH, IT><<<grid, TH, 0, g_stream>>>(a);
+    } else {
+        k_rank_pass<uint32_t, 4, kOrder, GRP, TH, IT><<<grid, TH, 0, g_stream>>>(a);
+    }
+    LAUNCHCHECK();
+}
+
+// One grouped pass.
+template <int TH, int IT>
+static void launch_grouped(const PassArgs &a, int64_t tiles, bool dbl, bool last) {
+    const dim3 grid((unsigned)tiles);
+    if (!last) return launch_order<true, TH, IT>(a, grid, dbl);
+    if (dbl) k_rank_pass<uint64_t, 0, kDirect, true, TH, IT><<<grid, TH, 0, g_stream>>>(a);
+    else k_rank_pass<uint32_t, 0, kDirect, true, TH, IT><<<grid, TH, 0, g_stream>>>(a);
+    LAUNCHCHECK();
+}
+
+// Up to this many keys the tiles' counts are grouped (no column scans), pass
+// 0 runs without waiting for the host, and the last pass stores the ranks
+// directly: one scattered 4-byte store per key, which stays in the caches
+// while the result is small, in place of the inverse's four or five launches.
+// us per call against the column scans and the partitioned inverse: 17000
+// ints 96 -> 44, 250000 101 -> 51, 10^6 116 -> 72, 3 10^6 152 -> 114, 5 10^6
+// 191 -> 171, 8 10^6 246 -> 236; 250000 doubles 182 -> 105, 3 10^6 303 -> 247,
+// 8 10^6 620 -> 592.  Above, a pass would add up more than kRankGroups
+// groups per tile, and the scattered stores miss the caches.
+constexpr int64_t kRankDirectMax = (int64_t)kRankGroups * kRankGroup * kRankTile;
+// Up to this many keys tiles are small: 250000 ints 51 against 57 us, 500000
+// 57 against 62, but 10^6 75 against 72.
+constexpr int64_t kRankSmallMax = (int64_t)1 << 19;
+
 void rank_run(int *rank, const void *s, int64_t n, bool dbl, bool up, const void *sd, int64_t m, void *scratch) {
     if (n <= 0) return;
     if (!scratch) usage_error("rank called without scratch");
@@ -878,8 +1008,6 @@ void rank_run(int *rank, const void *s, int64_t n, bool dbl, bool up, const void
     char *b = (char *)scratch;
     unsigned *hist = (unsigned *)(b + L.hist);
     unsigned *starts = (unsigned *)(b + L.starts);
-    unsigned *tile_ofs = (unsigned *)(b + L.status);
-    uint64_t *scan_status = (uint64_t *)(b + L.scan_status);
     const bool segmented = sd != nullptr && m > 1;
     if (!segmented && n <= (dbl ? kBlockRankMax8 : kBlockRankMax4)) {
         if (dbl) launch_rank_block<uint64_t, kBlockRankMax8 / kBlockRankThreads>(s, (int)n, up, rank);
@@ -894,23 +1022,56 @@ void rank_run(int *rank, const void *s, int64_t n, bool dbl, bool up, const void
         while (mm > 0) { seg_passes++; mm >>= 8; }
     }
     const int total = key_passes + seg_passes;
-    const int64_t tiles = (n + kRankTile - 1) / kRankTile;
 
     const bool chain = kRankChain && n < (int64_t)kChainMask;
-    const int64_t sw = tile_scan_status_words(tiles);
-    if (!g_hist_host) HIPCHECK(hipHostMalloc(&g_hist_host, 4 * 12 * kRadix, hipHostMallocDefault));
     const bool aligned = ((uintptr_t)s & 15) == 0;
-    int g = grid_for(n, kBlock * 16);
-    if (g > 2048) g = 2048;
+    // Short vectors are ranked in small tiles, whose counts lie in the
+    // inverse's scratch (n bytes and n / 32 per pass of its 16 n): a direct
+    // inverse needs none.
+    const bool grouped = !chain && n <= kRankDirectMax;
+    const bool small = grouped && n <= kRankSmallMax;
+    static_assert(kRankSmallMax <= (int64_t)kRankGroups * kRankGroup * kRankSmallThreads * kRankSmallItems,
+                  "small tiles are grouped");
+    const int tile = small ? kRankSmallThreads * kRankSmallItems : kRankTile;
+    const int64_t tiles = (n + tile - 1) / tile;
+    const int64_t ngroups = (tiles + kRankGroup - 1) / kRankGroup;
+    const int64_t sw = tile_scan_status_words((n + kRankTile - 1) / kRankTile);
+    unsigned *tile_ofs = (unsigned *)(b + L.status);
+    uint64_t *scan_status = (uint64_t *)(b + L.scan_status);
+    uint32_t *or_parts = (uint32_t *)(b + L.orparts);
+    unsigned *groups = (unsigned *)scan_status;             // ngroups x 256 per pass, in the space of its scan status
+    if (small) {
+        tile_ofs = (unsigned *)(b + L.invert);
+        groups = tile_ofs + kRadix * tiles;
+        or_parts = groups + 12 * kRadix * ngroups;
+    }
     int gs = grid_for(m, kBlock);
     if (gs > 4096) gs = 4096;
     bool runs[12] = {};
-    // The speculative first histogram (below): pass 0's tile counts, column
-    // scanned with its own status region (index 13).
     unsigned *tile_ofs2 = (unsigned *)(b + L.status2);
     InvertFirstPass inv{};
-    bool spec = false;
+    void *keys[2] = {b + L.keysA, b + L.keysB};
+    int *idxs[2] = {(int *)(b + L.idxA), (int *)(b + L.idxB)};
+    int cur = -1;   // buffer holding the current (keys, idx); -1 = original input
+    int kshift = 0;  // the stored keys are the transformed keys >> kshift
+    int kbytes = dbl ? 8 : 4;
+
+    PassArgs a0{};
+    a0.n = n;
+    a0.up = up;
+    a0.seg = seg;
+    a0.source = dbl ? 1 : 0;
+    a0.src = s;
+    a0.vec4 = !dbl && aligned;
+    a0.err = device_error_word();
+    a0.tile_ofs = tile_ofs;
+    a0.groups = grouped ? groups : nullptr;
+    a0.ngroups = ngroups;
+    bool first_counted = false;             // pass 0's tile counts are taken and scanned
     if (chain) {
+        if (!g_hist_host) HIPCHECK(hipHostMalloc(&g_hist_host, 4 * 12 * kRadix, hipHostMallocDefault));
+        int g = grid_for(n, kBlock * 16);
+        if (g > 2048) g = 2048;
         // chained passes need every digit's start up front: full histograms
         fill_u32(hist, 0, 12 * kRadix);
         if (dbl) k_key_hist<true><<<g, kBlock, 0, g_stream>>>(s, n, up, aligned, hist);
@@ -933,8 +1094,9 @@ void rank_run(int *rank, const void *s, int64_t n, bool dbl, bool up, const void
         // Pass 0's tile counts, which nearly always serve, also give the
         // keys' OR words; k_or_post posts which passes run to the host.
         // Behind it the device clears the scan status regions and the
-        // inverse's counters and column-scans pass 0's counts, covering the
-        // host's wait and its next launches.
+        // inverse's counters and column-scans pass 0's counts (or, with
+        // grouped tiles, runs pass 0), covering the host's wait and its next
+        // launches.
         unsigned *words = hist;
         static_assert(kOrCopies * kOrWords * kOrStride <= 12 * kRadix, "the OR words fit the histogram space");
         if (seg_passes) {
@@ -942,42 +1104,47 @@ void rank_run(int *rank, const void *s, int64_t n, bool dbl, bool up, const void
             k_seg_or<<<gs, kBlock, 0, g_stream>>>(seg.lens, m, words);
             LAUNCHCHECK();
         }
-        PassArgs a0{};
-        a0.n = n;
-        a0.up = up;
-        a0.seg = seg;
-        a0.source = dbl ? 1 : 0;
-        a0.src = s;
-        a0.shift = 0;
-        a0.vec4 = !dbl && aligned;
-        a0.err = device_error_word();
-        uint32_t *or_parts = (uint32_t *)(b + L.orparts);
-        if (dbl)
-            k_rank_hist<uint64_t, false, true><<<(unsigned)tiles, kRankThreads, 0, g_stream>>>(a0, tile_ofs, nullptr,
-                                                                                              or_parts);
-        else
-            k_rank_hist<uint32_t, false, true><<<(unsigned)tiles, kRankThreads, 0, g_stream>>>(a0, tile_ofs, nullptr,
-                                                                                              or_parts);
-        LAUNCHCHECK();
+        // the group counts of every pass
+        if (grouped) fill_u32(groups, 0, (int64_t)total * kRadix * ngroups);
+        if (small) launch_hist<kRankSmallThreads, kRankSmallItems, false, true>(a0, tiles, dbl, tile_ofs, nullptr, or_parts);
+        else launch_hist<kRankThreads, kRankItems, false, true>(a0, tiles, dbl, tile_ofs, nullptr, or_parts);
         const unsigned long long seq = mailbox_next();
         k_or_post<<<1, kOrPostThreads, 0, g_stream>>>(or_parts, tiles, seg_passes ? words : nullptr, key_passes,
                                                       seg_passes, mailbox_device(), seq);
         LAUNCHCHECK();
-        fill_u32(scan_status, 0, 2 * sw * 14);      // status regions: 12 passes, the inverse's counts, pass 0's
-        tile_scan(tile_ofs, tiles, nullptr, scan_status + 13 * sw, true, starts);
-        spec = true;
         // An unsegmented rank whose inverse takes two or more partition
-        // passes runs the first of them inside its last pass (FUSE): the pass
-        // knows every element's sorted position as it places it, so the
+        // passes runs the first of them inside its last pass (kFuse): the
+        // pass knows every element's sorted position as it places it, so the
         // order is never written and read back.
-        if (!segmented) inv = partition_invert_begin(n, b + L.invert);
+        if (!segmented && !grouped) inv = partition_invert_begin(n, b + L.invert);
+        if (grouped) {
+            // Pass 0 runs whether or not its digit varies (a pass over one
+            // digit keeps the order), so that the device works through the
+            // host's wait.
+            PassArgs a = a0;
+            a.keys_out = keys[0];
+            a.oshift = dbl ? 0 : 8;
+            a.idx_out = idxs[0];
+            a.kout = kbytes;
+            if (small) launch_grouped<kRankSmallThreads, kRankSmallItems>(a, tiles, dbl, false);
+            else launch_grouped<kRankThreads, kRankItems>(a, tiles, dbl, false);
+            cur = 0;
+            kshift = a.oshift;
+        } else {
+            fill_u32(scan_status, 0, 2 * sw * 14);   // status regions: 12 passes, the inverse's counts, pass 0's
+            tile_scan(tile_ofs, tiles, nullptr, scan_status + 13 * sw, true, starts);
+            first_counted = true;
+        }
         const unsigned long long mask = mailbox_wait(seq);
         for (int p = 0; p < total; p++) runs[p] = (mask >> p) & 1u;
     }
     int run[12], nrun = 0;
-    for (int p = 0; p < total; p++)
-        if (runs[p]) run[nrun++] = p;
-    if (nrun == 0) {
+    bool any = false;
+    for (int p = 0; p < total; p++) {
+        any = any || runs[p];
+        if (runs[p] && !(grouped && p == 0)) run[nrun++] = p;
+    }
+    if (!any) {
         k_rank_identity<<<grid_for(n, kBlock * 4), kBlock, 0, g_stream>>>(rank, n, seg, segmented);
         LAUNCHCHECK();
         return;
@@ -987,27 +1154,19 @@ void rank_run(int *rank, const void *s, int64_t n, bool dbl, bool up, const void
     for (int i = 0; i < nrun; i++) if (run[i] < key_passes) last_key_run = i;
     // pass 0's speculative counts serve when pass 0 runs, unless it is also
     // the fused last pass, which counts the inverse's children as well
-    spec = spec && run[0] == 0 && !(inv.pairs && nrun == 1);
+    first_counted = first_counted && run[0] == 0 && !(inv.pairs && nrun == 1);
 
     // Chained passes: per-digit counts below 2^30 (n < 2^30); one set of
     // words for all passes (alternating state sets) and a tile counter per
     // pass, contiguous and cleared together.
     unsigned *tickets = (unsigned *)(b + L.counters);
     if (chain) fill_u32(tickets, 0, (L.status - L.counters) / 4 + kRadix * tiles);
-    void *keys[2] = {b + L.keysA, b + L.keysB};
-    int *idxs[2] = {(int *)(b + L.idxA), (int *)(b + L.idxB)};
-    int cur = -1;   // buffer holding the current (keys, idx); -1 = original input
-    int kshift = 0;  // the stored keys are the transformed keys >> kshift
-    int kbytes = dbl ? 8 : 4;
+    bool done = false;
     for (int i = 0; i < nrun; i++) {
         const int p = run[i];
         const int out = cur == 0 ? 1 : 0;
-        PassArgs a;
-        a.n = n;
-        a.up = up;
-        a.seg = seg;
+        PassArgs a = a0;
         a.starts = starts + p * kRadix;
-        a.tile_ofs = tile_ofs;
         a.chain = chain ? (uint32_t *)tile_ofs : nullptr;
         a.ticket = tickets + i;
         a.parity = i & 1;
@@ -1024,7 +1183,6 @@ void rank_run(int *rank, const void *s, int64_t n, bool dbl, bool up, const void
         a.vec4 = a.source == 5 || a.source == 6 || ((a.source == 0 || a.source == 2) && ((uintptr_t)a.src & 15) == 0);
         a.keys_out = i < last_key_run ? keys[out] : nullptr;
         a.kout = kbytes;
-        a.oshift = 0;
         if (a.keys_out && !dbl) {
             // the next pass that reads keys is run[i + 1] (key passes come first)
             const int nshift = 8 * run[i + 1];
@@ -1033,49 +1191,43 @@ void rank_run(int *rank, const void *s, int64_t n, bool dbl, bool up, const void
             a.oshift = nshift - kshift;
         }
         a.idx_out = idxs[out];
-        a.err = device_error_word();
-        const bool fuse = inv.pairs && i + 1 == nrun;
+        if (grouped) a.groups = groups + (int64_t)p * kRadix * ngroups;
+        const bool last = i + 1 == nrun;
+        const bool fuse = inv.pairs && last;
         a.pairs = fuse ? inv.pairs : nullptr;
         a.tile_ofs2 = tile_ofs2;
         a.clog = inv.clog;
-        if (!chain && !(i == 0 && spec)) {
-            if (fuse) {
-                if (dbl) k_rank_hist<uint64_t, true><<<(unsigned)tiles, kRankThreads, 0, g_stream>>>(a, tile_ofs, tile_ofs2);
-                else k_rank_hist<uint32_t, true><<<(unsigned)tiles, kRankThreads, 0, g_stream>>>(a, tile_ofs, tile_ofs2);
-            } else {
-                if (dbl) k_rank_hist<uint64_t, false><<<(unsigned)tiles, kRankThreads, 0, g_stream>>>(a, tile_ofs, nullptr);
-                else k_rank_hist<uint32_t, false><<<(unsigned)tiles, kRankThreads, 0, g_stream>>>(a, tile_ofs, nullptr);
-            }
-            LAUNCHCHECK();
+        a.rank = rank;
+        a.rel = segmented;
+        if (!chain && !(i == 0 && first_counted)) {
+            if (fuse) launch_hist<kRankThreads, kRankItems, true, false>(a, tiles, dbl, tile_ofs, tile_ofs2, nullptr);
+            else if (small) launch_hist<kRankSmallThreads, kRankSmallItems, false, false>(a, tiles, dbl, tile_ofs, nullptr, nullptr);
+            else launch_hist<kRankThreads, kRankItems, false, false>(a, tiles, dbl, tile_ofs, nullptr, nullptr);
             // the column scan also leaves the digits' starts (the scan of its totals)
-            tile_scan(tile_ofs, tiles, nullptr, scan_status + i * sw, true, starts + p * kRadix);
+            if (!grouped) tile_scan(tile_ofs, tiles, nullptr, scan_status + i * sw, true, starts + p * kRadix);
             // the children's totals go to the inverse's counters
             if (fuse) tile_scan(tile_ofs2, tiles, inv.cnt, scan_status + 12 * sw, true);
         }
-        const dim3 grid((unsigned)tiles), block(kRankThreads);
-        if (fuse) {
-            if (dbl) k_rank_pass<uint64_t, 0, true><<<grid, block, 0, g_stream>>>(a);
-            else k_rank_pass<uint32_t, 0, true><<<grid, block, 0, g_stream>>>(a);
-        } else if (dbl) {
-            if (a.keys_out) k_rank_pass<uint64_t, 8><<<grid, block, 0, g_stream>>>(a);
-            else k_rank_pass<uint64_t, 0><<<grid, block, 0, g_stream>>>(a);
-        } else if (!a.keys_out) {
-            k_rank_pass<uint32_t, 0><<<grid, block, 0, g_stream>>>(a);
-        } else if (a.kout == 1) {
-            k_rank_pass<uint32_t, 1><<<grid, block, 0, g_stream>>>(a);
-        } else if (a.kout == 2) {
-            k_rank_pass<uint32_t, 2><<<grid, block, 0, g_stream>>>(a);
+        if (small) {
+            launch_grouped<kRankSmallThreads, kRankSmallItems>(a, tiles, dbl, last);
+        } else if (grouped) {
+            launch_grouped<kRankThreads, kRankItems>(a, tiles, dbl, last);
+        } else if (fuse) {
+            if (dbl) k_rank_pass<uint64_t, 0, kFuse, false><<<(unsigned)tiles, kRankThreads, 0, g_stream>>>(a);
+            else k_rank_pass<uint32_t, 0, kFuse, false><<<(unsigned)tiles, kRankThreads, 0, g_stream>>>(a);
+            LAUNCHCHECK();
         } else {
-            k_rank_pass<uint32_t, 4><<<grid, block, 0, g_stream>>>(a);
+            launch_order<false, kRankThreads, kRankItems>(a, dim3((unsigned)tiles), dbl);
         }
-        LAUNCHCHECK();
         if (a.keys_out) {
             kshift += a.oshift;
             kbytes = a.kout;
         }
         cur = out;
+        done = grouped && last;
     }
     // rank = inverse of the final order
+    if (done) return;
     if (inv.pairs) partition_invert_finish(rank, n, b + L.invert);
     else partition_invert(rank, idxs[cur], n, segmented ? sd : nullptr, m, b + L.invert);
 }

@@ -55,3 +55,48 @@ def test_short_double_ranks(cv, n):
     check(cv, rng.integers(-2, 3, n).astype(np.float64), "d", f"few {n}")
     special = np.array([0.0, -0.0, np.inf, -np.inf, np.nan, -np.nan, 5e-324, 1.7e308])
     check(cv, special[rng.integers(0, special.size, n)], "d", f"special {n}")
+
+
+# The ends of each rule above one workgroup: small tiles (to 2^19 keys),
+# grouped tile counts and direct ranks (to 2^23), then the column scans and
+# the inverse's first pass inside the last one.
+LONG = [16385, 32769, (1 << 19) - 1, 1 << 19, (1 << 19) + 1, (1 << 21) + 1, 1 << 23, (1 << 23) + 1]
+
+
+@pytest.mark.parametrize("n", LONG)
+def test_rank_rules(cv, n):
+    import torch
+    rng = np.random.default_rng(n)
+    print("rank rules", n, flush=True)
+    for ty, x in (("z", rng.integers(-2 ** 31, 2 ** 31, n).astype(np.int32)), ("d", rng.uniform(-1, 1, n))):
+        s = torch.from_numpy(x).to(cv.device)
+        d = torch.empty(n, dtype=torch.int32, device=cv.device)
+        order = np.argsort(x, kind="stable")
+        want = np.empty(n, np.int32)
+        want[order] = np.arange(n, dtype=np.int32)
+        L = cv.lib
+        getattr(L, f"rku_lu{ty}")(d, s, n, cv.scratch(getattr(L, f"rku_lu{ty}_scratch")(n)))
+        eq(host(d), want, f"rank {ty} {n}")
+    assert cv.lib.cvlhip_check_device_errors() == 0
+
+
+@pytest.mark.parametrize("n", [20_001, (1 << 19) + 3, (1 << 21) + 5])
+def test_segmented_rank_rules(cv, n):
+    """Segment passes after the key passes, empty segments among them, and
+    keys all equal (only segment passes reorder anything, then nothing)."""
+    import torch
+    rng = np.random.default_rng(n)
+    lens = rng.geometric(1 / 40, size=n).astype(np.int64)
+    lens = lens[np.cumsum(lens) <= n]
+    lens = np.append(lens, n - lens.sum())
+    lens = np.insert(lens, [0, 5, lens.size // 2], 0).astype(np.int32)
+    sd = cv.segd(lens)
+    for kind in ("random", "equal", "low"):
+        x = {"random": rng.integers(-2 ** 31, 2 ** 31, n), "equal": np.full(n, 3), "low": rng.integers(0, 200, n)}[kind]
+        x = x.astype(np.int32)
+        s = torch.from_numpy(x).to(cv.device)
+        d = torch.empty(n, dtype=torch.int32, device=cv.device)
+        print("segmented rank", n, kind, flush=True)
+        cv.lib.rku_lez(d, s, sd, n, lens.size, cv.scratch(cv.lib.rku_lez_scratch(n, lens.size)))
+        eq(host(d), O.rank(x, True, lens), f"segmented rank {kind} {n}")
+    assert cv.lib.cvlhip_check_device_errors() == 0

@@ -19,6 +19,9 @@
 //   block scatter     One workgroup per destination block scatters its
 //                     pairs into LDS and writes the block out in order.
 //
+// Vectors that stay in the caches are scattered directly (k_permute_direct):
+// there the passes' launches cost more than the scattered stores.
+//
 // Pairs whose index is out of range, or that overflow their bucket (the
 // indices were not a permutation), are dropped and raise the device error
 // word; destination positions nobody wrote keep their old contents.
@@ -500,6 +503,92 @@ __global__ __launch_bounds__(kPartThreads) void k_block_scatter(IndexSource src,
         if ((s_mask[o >> 5] >> (o & 31)) & 1u) d[base + o] = s_out[o];
 }
 
+// Direct permute of vectors that stay in the caches: every value is stored
+// where its index says, one scattered store each, in two launches (the
+// counters' clear is the other) instead of five to seven.  The indices aimed
+// at each destination block are still counted, per workgroup in LDS and then
+// with one atomic per block, so that indices that are no permutation raise
+// the device error word as they do when they overflow a block of the
+// partition.  Bound by the scattered stores (about 70 G/s) and by those
+// atomics: workgroups hold as many elements as still leave every CU one
+// (2 10^6 ints: 55 us with 1024 elements per workgroup, 31 with 4096, 29 with
+// 8192).  us against the partition: ints 9000 29 -> 9, 250000 22 -> 8, 10^6
+// 26 -> 17, 2 10^6 31.4 -> 29.2, but 4 10^6 57 -> 56 and 8 10^6 90 -> 105;
+// doubles 10^6 30 -> 18, 4 10^6 77 -> 58, 8 10^6 135 -> 110, 16 10^6 269 -> 227.
+constexpr int kDirectLog4 = 21, kDirectLog8 = 24;
+template <class T>
+constexpr int direct_log() { return sizeof(T) == 4 ? kDirectLog4 : kDirectLog8; }
+
+template <class T, int TH, int ITEMS>
+__global__ __launch_bounds__(TH) void k_permute_direct(IndexSource src, const T *__restrict__ in_val,
+                                                                   T *__restrict__ d, int64_t n,
+                                                                   unsigned *__restrict__ cnt,
+                                                                   unsigned *__restrict__ err) {
+    constexpr int BLOG = blk_log<T>();
+    constexpr int kBlocks = 1 << (direct_log<T>() - BLOG);
+    static_assert(ITEMS % kPartV == 0, "items per thread come in runs of kPartV");
+    __shared__ unsigned s_hist[kBlocks];
+    const int tid = threadIdx.x;
+    const int blocks = (int)((n - 1) >> BLOG) + 1;
+    for (int i = tid; i < blocks; i += TH) s_hist[i] = 0;
+    __syncthreads();
+    const int64_t lo = (int64_t)blockIdx.x * TH * ITEMS;
+    int64_t q[ITEMS];
+    T v[ITEMS];
+#pragma unroll
+    for (int g = 0; g < ITEMS / kPartV; g++) {
+        const int64_t e0 = lo + ((int64_t)g * TH + tid) * kPartV;
+        if (src.vec && e0 + kPartV <= n) {
+            int qi[kPartV];
+            T vi[kPartV];
+            load4(src.p + e0, qi);
+            if (src.vmode == 0) load4(in_val + e0, vi);
+#pragma unroll
+            for (int c = 0; c < kPartV; c++) {
+                q[g * kPartV + c] = qi[c];
+                v[g * kPartV + c] = src.vmode == 0 ? vi[c] : (T)(e0 + c);
+            }
+        } else {
+#pragma unroll
+            for (int c = 0; c < kPartV; c++) {
+                const int64_t e = e0 + c;
+                q[g * kPartV + c] = 0;
+                v[g * kPartV + c] = T(0);
+                if (e < n) {
+                    q[g * kPartV + c] = src.at(e);
+                    v[g * kPartV + c] = src.value(in_val, e);
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < ITEMS; j++) {
+        const int64_t e = lo + ((int64_t)(j / kPartV) * TH + tid) * kPartV + j % kPartV;
+        if (e >= n) continue;
+        if (q[j] >= 0 && q[j] < n) {
+            d[q[j]] = v[j];
+            atomicAdd(&s_hist[q[j] >> BLOG], 1u);
+        } else {
+            atomicOr(err, 1u);
+        }
+    }
+    __syncthreads();
+    for (int b = tid; b < blocks; b += TH) {
+        const unsigned c = s_hist[b];
+        if (!c) continue;
+        const int64_t left = n - ((int64_t)b << BLOG);
+        const unsigned size = left < ((int64_t)1 << BLOG) ? (unsigned)left : 1u << BLOG;
+        if (atomicAdd(cnt + b, c) + c > size) atomicOr(err, 1u);
+    }
+}
+
+template <class T, int TH, int ITEMS>
+static void launch_permute_direct(IndexSource src, const void *s, void *d, int64_t n, unsigned *cnt, unsigned *err) {
+    k_permute_direct<T, TH, ITEMS><<<(unsigned)grid_for(n, TH * ITEMS), TH, 0, g_stream>>>(src, (const T *)s, (T *)d, n, cnt,
+                                                                                         err);
+    LAUNCHCHECK();
+}
+
 static int64_t up256(int64_t b) { return (b + 255) & ~(int64_t)255; }
 
 // Scratch: two (idx, val) buffers of n pairs and one counter array per
@@ -616,6 +705,16 @@ static void partition_later_levels(const PartLayout<T> &L, IndexSource src, void
 template <class T>
 static void run_partition(void *d, const void *s, IndexSource src, int64_t n, void *scratch) {
     unsigned *err = device_error_word();
+    if (n > ((int64_t)1 << blk_log<T>()) && n <= ((int64_t)1 << direct_log<T>())) {
+        if (!scratch) { usage_error("permute called without scratch"); return; }
+        unsigned *cnt = (unsigned *)scratch;
+        fill_u32(cnt, 0, ((n - 1) >> blk_log<T>()) + 1);
+        if (n <= (1 << 18)) launch_permute_direct<T, 256, 4>(src, s, d, n, cnt, err);
+        else if (n <= (1 << 19)) launch_permute_direct<T, 1024, 4>(src, s, d, n, cnt, err);
+        else if (n <= (1 << 23)) launch_permute_direct<T, 1024, 8>(src, s, d, n, cnt, err);
+        else launch_permute_direct<T, 1024, 16>(src, s, d, n, cnt, err);
+        return;
+    }
     const PartLayout<T> L(n, scratch);
     L.clear();
     if (L.levels == 0) {
@@ -637,16 +736,6 @@ static void run_partition(void *d, const void *s, IndexSource src, int64_t n, vo
         k_part_hist<<<(unsigned)L.grid0, kPartThreads, 0, g_stream>>>(src, n, clog, hist);
         LAUNCHCHECK();
         tile_scan(hist, L.grid0, cnt, L.status0, true);
-    }
-    if (L.levels == 1) {
-        k_partition<T, true, Local16<T>><<<(unsigned)L.grid0, kPartThreads, 0, g_stream>>>(
-            src, Pairs<T>{}, (const T *)s, L.local[0], n, plog, clog, tpr, nullptr, cnt, hist, err, lb, lb_ctr);
-        LAUNCHCHECK();
-        const int64_t blocks = ((n - 1) >> blk_log<T>()) + 1;
-        k_block_scatter<T, false, Local16<T>><<<(unsigned)blocks, kPartThreads, 0, g_stream>>>(
-            src, L.local[0], nullptr, (T *)d, n, cnt, err);
-        LAUNCHCHECK();
-        return;
     }
     k_partition<T, true><<<(unsigned)L.grid0, kPartThreads, 0, g_stream>>>(
         src, Pairs<T>{}, (const T *)s, L.buf[0], n, plog, clog, tpr, nullptr, cnt, hist, err, lb, lb_ctr);

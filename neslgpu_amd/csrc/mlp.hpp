@@ -58,27 +58,69 @@ __host__ __device__ inline int max_len_class(const uint32_t *segs) {
     return c;
 }
 
+// Parameters staged in LDS for mlp_pick_wave: rows of W2 and W3 one word
+// longer than in the array, so that the lanes of a step (one row each) read
+// different banks; W1's rows are of odd length already.
+constexpr int kPitch = kH + 1;
+constexpr int kLB2 = kW2 + kH * kPitch, kLW3 = kLB2 + kH, kLB3 = kLW3 + kA * kPitch, kLdsParams = kLB3 + kA;
+__device__ __forceinline__ int lds_param(int i) {
+    if (i < kW2) return i;
+    if (i < kB2) return i + (i - kW2) / kH;
+    if (i < kW3) return i - kB2 + kLB2;
+    if (i < kB3) return i - kW3 + kLW3 + (i - kW3) / kH;
+    return i - kB3 + kLB3;
+}
+// Stage the parameters (THREADS threads, which then need a barrier), all
+// loads in flight together.
+template <int THREADS>
+__device__ __forceinline__ void stage_params(const float *__restrict__ params, float *s_P) {
+    constexpr int PER = (kParams + THREADS - 1) / THREADS;
+    float v[PER];
+#pragma unroll
+    for (int k = 0; k < PER; k++) {
+        const int i = k * THREADS + (int)threadIdx.x;
+        v[k] = i < kParams ? params[i] : 0.f;
+    }
+#pragma unroll
+    for (int k = 0; k < PER; k++) {
+        const int i = k * THREADS + (int)threadIdx.x;
+        if (i < kParams) s_P[lds_param(i)] = v[k];
+    }
+}
+
+// The value x has in lane i (the same i in every lane).
+__device__ __forceinline__ float lane_value(float x, int i) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), i));
+}
+
 // Forward pass of one feature vector by one whole wave (lane i holds
 // feature i); every lane returns the index of the smallest prediction among
-// the admitted schedules (the first one on ties).  Values move between lanes with shuffles only, and
-// sums run in index order, so the same parameters and features always give
-// the same pick.
+// the admitted schedules (the first one on ties).  P: the staged parameters.
+// Sums run in index order, so the same parameters and features always give
+// the same pick.  Bound by latency: the steps are unrolled, so that their
+// LDS reads are in flight together, and take the other lanes' values from
+// registers (v_readlane) instead of LDS shuffles (with the launch that waits
+// for the pick: 9.3 -> 4.6 us).
 __device__ __forceinline__ int mlp_pick_wave(const float *__restrict__ P, float feature_of_lane, unsigned admitted) {
     const int lane = lane_id();
     const int j1 = lane < kH ? lane : kH - 1;       // lanes past a layer's width compute a copy
     float a = P[kB1 + j1];
-    for (int i = 0; i < kF; i++) a += P[kW1 + j1 * kF + i] * shfl(feature_of_lane, i);
+#pragma unroll
+    for (int i = 0; i < kF; i++) a += P[kW1 + j1 * kF + i] * lane_value(feature_of_lane, i);
     const float h1 = a > 0.f ? a : 0.f;
-    a = P[kB2 + j1];
-    for (int i = 0; i < kH; i++) a += P[kW2 + j1 * kH + i] * shfl(h1, i);
+    a = P[kLB2 + j1];
+#pragma unroll
+    for (int i = 0; i < kH; i++) a += P[kW2 + j1 * kPitch + i] * lane_value(h1, i);
     const float h2 = a > 0.f ? a : 0.f;
     const int j3 = lane < kA ? lane : kA - 1;
-    a = P[kB3 + j3];
-    for (int i = 0; i < kH; i++) a += P[kW3 + j3 * kH + i] * shfl(h2, i);
+    a = P[kLB3 + j3];
+#pragma unroll
+    for (int i = 0; i < kH; i++) a += P[kLW3 + j3 * kPitch + i] * lane_value(h2, i);
     int best = 0;                                   // flat8 is always admitted
-    float by = shfl(a, 0);
+    float by = lane_value(a, 0);
+#pragma unroll
     for (int k = 1; k < kA; k++) {
-        const float v = shfl(a, k);
+        const float v = lane_value(a, k);
         if (((admitted >> k) & 1u) && v < by) { by = v; best = k; }
     }
     return best;

@@ -5,12 +5,12 @@
 // offsets (a scan of the lengths), the list of non-empty segments, the head
 // bitmap and the per-word head counts.  It runs once per descriptor; every
 // segmented kernel then finds boundaries from the bitmap.  Small
-// descriptors are built by one workgroup, larger ones by two single-pass
-// look-back kernels.
+// descriptors are built by one workgroup, larger ones by three kernels (sums
+// of the lengths per tile; offsets; bitmap and head counts), none of which
+// waits for another workgroup.
 #include "cvl_hip.hpp"
 #include "segd.hpp"
 #include "scan.hpp"
-#include "lookback.hpp"
 #include "mlp.hpp"
 #include "../../include/cvl.h"
 #include "../../include/cvl_hip_ext.h"
@@ -46,25 +46,38 @@ static int g_sched_enabled = sched_enabled_at_load();
 
 constexpr int kHist = 2 * kLenClasses;
 
+// A workgroup's histogram is kept in kHistCopies copies, one for every
+// kHistCopies-th lane, since the lanes of a wave mostly add to the same few
+// classes and LDS atomics on one word take turns (k_segd_offsets 5.1 -> 4.5 us
+// at 16384 lengths).
+constexpr int kHistCopies = 8;
 __device__ __forceinline__ void hist_add(unsigned *h, unsigned len) {
     if (len == 0) return;
     int c = 31 - __clz(len);
     if (c >= kLenClasses) c = kLenClasses - 1;
-    atomicAdd(h + c, len);
-    atomicAdd(h + kLenClasses + c, 1u);
+    const int copy = threadIdx.x % kHistCopies;
+    atomicAdd(h + c * kHistCopies + copy, len);
+    atomicAdd(h + (kLenClasses + c) * kHistCopies + copy, 1u);
+}
+__device__ __forceinline__ unsigned hist_get(const unsigned *h, int i) {
+    unsigned s = 0;
+#pragma unroll
+    for (int k = 0; k < kHistCopies; k++) s += h[i * kHistCopies + k];
+    return s;
 }
 
-// Waves 0..3 of a workgroup of at least 256 threads each pick the schedule
+// Waves 0..3 of a workgroup of THREADS (at least 256) each pick the schedule
 // of one kind of operation (sched_slot order) from the histogram `hist`;
 // thread 0 stores the picks in the header.  Every thread of the workgroup
 // must call it.
+template <int THREADS>
 __device__ void sched_pick_block(SegdHeader *hdr, int64_t n, int64_t m, const unsigned *hist, unsigned *s_pick) {
     // The network's parameters and the histogram are staged in LDS with
     // one coalesced pass first, so the forward passes wait for memory once
     // instead of once per layer.
-    __shared__ float s_P[kParams];
+    __shared__ float s_P[kLdsParams];
     __shared__ unsigned s_h[kHist];
-    for (int i = threadIdx.x; i < kParams; i += blockDim.x) s_P[i] = g_sched_params[i];
+    stage_params<THREADS>(g_sched_params, s_P);
     if (threadIdx.x < kHist) s_h[threadIdx.x] = hist[threadIdx.x];
     __syncthreads();
     const int w = threadIdx.x / kWave, lane = threadIdx.x % kWave;
@@ -116,10 +129,11 @@ __global__ __launch_bounds__(kSmallThreads) void k_segd_small(const int *__restr
     __shared__ unsigned s_wave[kSmallThreads / kWave];
     __shared__ unsigned s_total;
     __shared__ uint32_t s_heads[kSmallSegd + 8];
+    __shared__ unsigned s_hc[kHist * kHistCopies];
     __shared__ unsigned s_hist[kHist];
     __shared__ unsigned s_pick[4];
     const int tid = threadIdx.x;
-    if (tid < kHist) s_hist[tid] = 0u;     // ordered by the barriers of the scans below
+    if (tid < kHist * kHistCopies) s_hc[tid] = 0u;     // ordered by the barriers of the scans below
     unsigned len[kSmallPer], off[kSmallPer], pos[kSmallPer];
     unsigned lsum = 0, psum = 0;
 #pragma unroll
@@ -146,7 +160,7 @@ __global__ __launch_bounds__(kSmallThreads) void k_segd_small(const int *__restr
             if ((int)len[k] > 0) {
                 nz[pbase + pos[k]] = (int)g;
                 if (o >= 0 && (int64_t)o < n) atomicOr(&s_heads[o >> 5], 1u << (o & 31));
-                hist_add(s_hist, len[k]);
+                hist_add(s_hc, len[k]);
             }
         }
     }
@@ -157,8 +171,9 @@ __global__ __launch_bounds__(kSmallThreads) void k_segd_small(const int *__restr
         hdr->stats = kStatsMagic;
     }
     __syncthreads();
-    if (tid < kHist) hdr->hist[tid] = s_hist[tid];
-    if (pick) sched_pick_block(hdr, n, m, s_hist, s_pick);
+    if (tid < kHist) hdr->hist[tid] = s_hist[tid] = hist_get(s_hc, tid);
+    __syncthreads();
+    if (pick) sched_pick_block<kSmallThreads>(hdr, n, m, s_hist, s_pick);
     else if (tid == 0) hdr->sched = 0u;
     unsigned hc[kSmallPer], csum = 0;
 #pragma unroll
@@ -179,116 +194,193 @@ __global__ __launch_bounds__(kSmallThreads) void k_segd_small(const int *__restr
     if (tid == 0) wcnt[words] = (int)s_total;
 }
 
-// ---- larger descriptors: two single-pass look-back kernels
-// Pass 1 scans the lengths for (offset, number of non-empty segments
-// before) as one packed pair, writes offs, the lengths copy, nz and the head
-// bits; pass 2 scans the popcounts of the head words into wcnt.  With the
-// clears, four launches instead of a dozen.
-struct AddUs : AddU {
-    __device__ static unsigned sub(unsigned a, unsigned b) { return a - b; }
-};
+// ---- larger descriptors
+// k_segd_sums adds up each tile of kTile lengths; k_segd_offsets, whose tiles
+// add up the sums before them, writes offs, the lengths copy, nz, the
+// histogram and the first head count (wcnt) of each chunk of kChunk elements;
+// k_segd_words builds each chunk's bitmap words in LDS from the starts of
+// its segments and writes them with the other head counts.  No workgroup
+// waits for another, nothing is cleared first but the histogram, and the
+// bitmap is written once, without atomics.  Two look-back kernels behind a
+// clear, which waited across the chip and set the bits with atomics in
+// memory, took 21.1 us for 300007 lengths of 5 10^6 elements and 19.2 for
+// 16384 of about 500000, these three 13.8 and 12.6, most of it latency of
+// dependent loads.
+constexpr int kTileThreads = 512;
+constexpr int kTile = kTileThreads * 4;         // lengths per tile
+// Threads of k_segd_words: with 256, chunks of many short segments wait for
+// twice as many rounds of loads (16384 one-element segments: 7.3 against
+// 5.6 us).
+constexpr int kChunkThreads = 512;
+constexpr int kChunkWords = 256;                // bitmap words per workgroup of k_segd_words
+constexpr int kChunk = kChunkWords * 32;        // elements per chunk
+// Above this many tiles the sums are scanned by a kernel of their own
+// instead of being added up by every tile.
+constexpr int64_t kDirectTiles = 4 * kTileThreads;
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
 struct SegPair {                    // (sum of lengths mod 2^32) | (count of non-empty) << 32
     using T = uint64_t;
     __host__ __device__ static T neutral() { return 0; }
-    __host__ __device__ static T cvl_id() { return 0; }
     __device__ T operator()(T a, T b) const {
         return (uint64_t)(uint32_t)((uint32_t)a + (uint32_t)b) | (((a >> 32) + (b >> 32)) << 32);
     }
-    __device__ static T sub(T a, T b) {
-        return (uint64_t)(uint32_t)((uint32_t)a - (uint32_t)b) | (((a >> 32) - (b >> 32)) << 32);
-    }
+    __device__ static T of(unsigned len) { return (uint64_t)len | ((uint64_t)((int)len > 0) << 32); }
 };
 
-template <class Op>
-__device__ typename Op::T block_tile_prefix(typename Op::T x, typename Op::T *s_wave, typename Op::T *s_tilep,
-                                            uint64_t *status, int64_t tile, unsigned *err,
-                                            typename Op::T *excl_in_block) {
-    // returns the exclusive prefix of this thread's value over all earlier
-    // tiles and threads; *s_tilep receives the tile's inclusive total
-    using T = typename Op::T;
-    using St = TileStatus<T>;
-    const Op op;
-    const int tid = threadIdx.x, lane = tid % kWave, w = tid / kWave;
-    constexpr int W = kSmallThreads / kWave;
-    const T inc = wave_inclusive_scan(x, op);
-    if (lane == kWave - 1) s_wave[w] = inc;
+// Sum over a workgroup of W waves, in every thread.
+template <int W>
+__device__ __forceinline__ uint64_t block_sum(uint64_t x, uint64_t *s_wave) {
+    const SegPair op;
+    const int w = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+    const uint64_t r = wave_reduce(x, op);
+    __syncthreads();                         // s_wave may still be read from a previous use
+    if (lane == 0) s_wave[w] = r;
     __syncthreads();
-    if (w == 0) {
-        T tv = Op::neutral();
-        T wp[W];
+    uint64_t tot = 0;
 #pragma unroll
-        for (int i = 0; i < W; i++) { wp[i] = tv; tv = op(tv, s_wave[i]); }
-        T P = Op::neutral();
-        if (tile == 0) {
-            if (lane == 0) St::publish(status, 0, kPrefix, tv);
-        } else {
-            if (lane == 0) St::publish(status, tile, kAggregate, tv);
-            P = lookback(status, tile, op, err);
-            if (lane == 0) St::publish(status, tile, kPrefix, op(P, tv));
-        }
-        if (lane == 0) {
-#pragma unroll
-            for (int i = 0; i < W; i++) s_wave[i] = op(P, wp[i]);
-            *s_tilep = op(P, tv);
-        }
-    }
-    __syncthreads();
-    *excl_in_block = Op::sub(inc, x);
-    return op(s_wave[w], *excl_in_block);
+    for (int i = 0; i < W; i++) tot = op(tot, s_wave[i]);
+    return tot;
 }
 
-// The header's histogram is cleared before the launch; every tile adds its
-// segments' counts to it.
-__global__ __launch_bounds__(kSmallThreads) void k_segd_offsets(const int *__restrict__ lens_in, SegdHeader *hdr,
-                                                                 int *lens, int *offs, int *nz, uint32_t *heads,
-                                                                 int64_t n, int64_t m, uint64_t *status,
-                                                                 unsigned *counter, unsigned *err) {
-    __shared__ unsigned s_tile;
-    __shared__ uint64_t s_wave[kSmallThreads / kWave];
-    __shared__ uint64_t s_total;
-    __shared__ int s_head[kSmallSegd];          // start of each non-empty segment of the tile, else -1
-    __shared__ unsigned s_hist[kHist];
-    const int tid = threadIdx.x;
-    if (tid < kHist) s_hist[tid] = 0u;
-    if (tid == 0) s_tile = atomicAdd(counter, 1u);
-    __syncthreads();
-    const int64_t tile = s_tile;
-    const int64_t g0 = tile * kSmallSegd + (int64_t)tid * kSmallPer;
-    unsigned len[kSmallPer];
-    uint64_t loc[kSmallPer], sum = 0;
-    const SegPair op;
+// Four lengths of a tile from segment g0 on (0 past the last).
+__device__ __forceinline__ void load_lengths(const int *__restrict__ lens, int64_t g0, int64_t m, unsigned (&len)[4]) {
+    if (((uintptr_t)lens & 15) == 0 && g0 + 4 <= m) {
+        const i32x4 v = *(const i32x4 *)(lens + g0);
+        len[0] = (unsigned)v.x;
+        len[1] = (unsigned)v.y;
+        len[2] = (unsigned)v.z;
+        len[3] = (unsigned)v.w;
+    } else {
 #pragma unroll
-    for (int k = 0; k < kSmallPer; k++) {
-        const int64_t g = g0 + k;
-        len[k] = g < m ? (unsigned)lens_in[g] : 0u;
-        loc[k] = sum;
-        sum = op(sum, (uint64_t)len[k] | ((uint64_t)(g < m && (int)len[k] > 0) << 32));
+        for (int k = 0; k < 4; k++) len[k] = g0 + k < m ? (unsigned)lens[g0 + k] : 0u;
     }
-    uint64_t excl;
-    const uint64_t P = block_tile_prefix<SegPair>(sum, s_wave, &s_total, status, tile, err, &excl);
-    int o4[kSmallPer];
+}
+
+// parts[t]: the SegPair sum of tile t.  Workgroup 0 also clears the header
+// from its schedule word to the end of the histogram.
+__global__ __launch_bounds__(kTileThreads) void k_segd_sums(const int *__restrict__ lens, int64_t m,
+                                                             uint64_t *__restrict__ parts, SegdHeader *hdr) {
+    __shared__ uint64_t s_wave[kTileThreads / kWave];
+    const int tid = threadIdx.x;
+    if (blockIdx.x == 0) {
+        if (tid < kHist) hdr->hist[tid] = 0u;
+        if (tid == 0) hdr->sched = hdr->stats = 0u;
+    }
+    unsigned len[4];
+    load_lengths(lens, (int64_t)blockIdx.x * kTile + tid * 4, m, len);
+    const SegPair op;
+    uint64_t sum = 0;
 #pragma unroll
-    for (int k = 0; k < kSmallPer; k++) {
-        const int64_t g = g0 + k;
+    for (int k = 0; k < 4; k++) sum = op(sum, SegPair::of(len[k]));
+    const uint64_t tot = block_sum<kTileThreads / kWave>(sum, s_wave);
+    if (tid == 0) parts[blockIdx.x] = tot;
+}
+
+// Exclusive scan of the tile sums in place, one workgroup.
+__global__ __launch_bounds__(kSmallThreads) void k_segd_scan_sums(uint64_t *parts, int64_t tiles) {
+    constexpr int W = kSmallThreads / kWave;
+    __shared__ uint64_t s_wave[W];
+    const SegPair op;
+    const int tid = threadIdx.x, w = tid / kWave, lane = tid % kWave;
+    uint64_t carry = 0;
+    for (int64_t base = 0; base < tiles; base += kSmallThreads) {
+        const uint64_t x = base + tid < tiles ? parts[base + tid] : 0;
+        const uint64_t inc = wave_inclusive_scan(x, op);
+        __syncthreads();
+        if (lane == kWave - 1) s_wave[w] = inc;
+        __syncthreads();
+        uint64_t before = carry;
+#pragma unroll
+        for (int i = 0; i < W; i++) {
+            if (i < w) before = op(before, s_wave[i]);
+            carry = op(carry, s_wave[i]);
+        }
+        uint64_t ex = shfl_up1(inc);
+        if (lane == 0) ex = 0;
+        if (base + tid < tiles) parts[base + tid] = op(before, ex);
+    }
+}
+
+// `scanned`: parts holds exclusive sums, else the tiles' own.  Of wcnt it
+// writes the first word of each chunk and the last, the number of all heads.
+__global__ __launch_bounds__(kTileThreads) void k_segd_offsets(const int *__restrict__ lens_in, SegdHeader *hdr,
+                                                                int *lens, int *offs, int *nz,
+                                                                int *__restrict__ wcnt,
+                                                                const uint64_t *__restrict__ parts, int scanned,
+                                                                int64_t n, int64_t m) {
+    constexpr int W = kTileThreads / kWave;
+    __shared__ uint64_t s_wave[W];
+    __shared__ unsigned s_hist[kHist * kHistCopies];
+    const SegPair op;
+    const int tid = threadIdx.x, w = tid / kWave, lane = tid % kWave;
+    const int64_t tile = blockIdx.x;
+    const int64_t g0 = tile * kTile + tid * 4;
+    if (tid < kHist * kHistCopies) s_hist[tid] = 0u;   // ordered by the barriers below
+    unsigned len[4];
+    load_lengths(lens_in, g0, m, len);
+    // the tiles before this one
+    uint64_t P = 0;
+    if (scanned) {
+        P = parts[tile];
+    } else if (tile > 0) {
+        uint64_t s = 0;
+        for (int64_t i = tid; i < tile; i += kTileThreads) s = op(s, parts[i]);
+        P = block_sum<W>(s, s_wave);
+    }
+    uint64_t loc[4], sum = 0;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        loc[k] = sum;
+        sum = op(sum, SegPair::of(len[k]));
+    }
+    const uint64_t inc = wave_inclusive_scan(sum, op);
+    __syncthreads();
+    if (lane == kWave - 1) s_wave[w] = inc;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < W; i++)
+        if (i < w) P = op(P, s_wave[i]);
+    uint64_t ex = shfl_up1(inc);
+    if (lane == 0) ex = 0;
+    P = op(P, ex);
+    int o4[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
         const uint64_t q = op(P, loc[k]);
         o4[k] = (int)(uint32_t)q;
-        s_head[tid * kSmallPer + k] = (g < m && (int)len[k] > 0 && o4[k] >= 0 && (int64_t)o4[k] < n) ? o4[k] : -1;
-        if (g < m && (int)len[k] > 0) {
-            nz[q >> 32] = (int)g;
+        const bool live = g0 + k < m && (int)len[k] > 0;
+        if (live) {
+            nz[q >> 32] = (int)(g0 + k);
             hist_add(s_hist, len[k]);
         }
+        // the chunks that start after this segment's head and no later than
+        // its end: a lane's own few, or, for a long segment, its wave's work
+        int j = 0, j1 = 0;
+        if (live && o4[k] >= 0) {
+            const int64_t end = (int64_t)o4[k] + len[k];
+            j = o4[k] / kChunk + 1;
+            j1 = (int)((end < n - 1 ? end : n - 1) / kChunk) + 1;
+        }
+        const int rank = (int)(q >> 32) + 1;
+        const bool wide = j1 - j > 4;
+        if (!wide)
+            for (; j < j1; j++) wcnt[(int64_t)j * kChunkWords] = rank;
+        for (uint64_t rest = ballot(wide); rest; rest &= rest - 1) {
+            const int l = __builtin_ctzll(rest);
+            const int from = shfl(j, l), to = shfl(j1, l), r = shfl(rank, l);
+            for (int i = from + lane; i < to; i += kWave) wcnt[(int64_t)i * kChunkWords] = r;
+        }
     }
-    static_assert(kSmallPer == 4, "one 16-byte store per thread");
-    typedef int i32x4 __attribute__((ext_vector_type(4)));
     // (a descriptor in a CVL arena starts on an 8-byte unit: check)
     const bool a16 = (((uintptr_t)offs | (uintptr_t)lens) & 15) == 0;
-    if (a16 && g0 + kSmallPer <= m) {    // g0 is a multiple of 4
+    if (a16 && g0 + 4 <= m) {    // g0 is a multiple of 4
         *(i32x4 *)(offs + g0) = i32x4{o4[0], o4[1], o4[2], o4[3]};
         if (lens != lens_in) *(i32x4 *)(lens + g0) = i32x4{(int)len[0], (int)len[1], (int)len[2], (int)len[3]};
     } else {
 #pragma unroll
-        for (int k = 0; k < kSmallPer; k++) {
+        for (int k = 0; k < 4; k++) {
             if (g0 + k < m) {
                 offs[g0 + k] = o4[k];
                 if (lens != lens_in) lens[g0 + k] = (int)len[k];
@@ -296,91 +388,89 @@ __global__ __launch_bounds__(kSmallThreads) void k_segd_offsets(const int *__res
         }
     }
     __syncthreads();
-    if (tid < kHist && s_hist[tid]) atomicAdd(&hdr->hist[tid], s_hist[tid]);
-    // Head bits: wave w takes the tile's segments w*256 .. w*256+255, 64
-    // consecutive ones per round, ORs the bits of lanes whose heads share a
-    // bitmap word (segment starts increase with the segment index) and
-    // lets the first lane of each such run set them with one atomic.
-    {
-        const int w = tid / kWave, lane = tid % kWave;
-#pragma unroll
-        for (int k = 0; k < kSmallPer; k++) {
-            const int o = s_head[w * kWave * kSmallPer + k * kWave + lane];
-            int key = o >= 0 ? (o >> 5) : -1 - lane;       // an empty segment matches no neighbour
-            uint32_t v = o >= 0 ? 1u << (o & 31) : 0u;
-#pragma unroll
-            for (int d = 1; d < kWave; d <<= 1) {
-                const uint32_t vo = __shfl_down(v, d);
-                const int ko = __shfl_down(key, d);
-                if (lane + d < kWave && ko == key) v |= vo;
-            }
-            const int kp = __shfl_up(key, 1);
-            if (o >= 0 && (lane == 0 || kp != key)) atomicOr(heads + (o >> 5), v);
-        }
+    const bool only = gridDim.x == 1;             // one tile: k_segd_sums did not run
+    if (tid < kHist) {
+        const unsigned h = hist_get(s_hist, tid);
+        if (only) hdr->hist[tid] = h;
+        else if (h) atomicAdd(&hdr->hist[tid], h);
     }
-    if (tile == (int64_t)gridDim.x - 1 && tid == 0) {
-        offs[m] = (int)(uint32_t)s_total;
+    if (tile == (int64_t)gridDim.x - 1 && tid == kTileThreads - 1) {
+        const uint64_t all = op(P, sum);
+        offs[m] = (int)(uint32_t)all;
+        wcnt[(n + 31) >> 5] = (int)(all >> 32);
         hdr->n = n;
         hdr->m = m;
         hdr->stats = kStatsMagic;
+        if (only) hdr->sched = 0u;
     }
+    if (tile == 0 && tid == 0 && n > 0) wcnt[0] = 0;
 }
 
-// With `pick`, the launch has one workgroup more than tiles, and that last
-// workgroup picks the schedules from the histogram k_segd_offsets completed,
-// beside the tiles instead of after one of them.
-__global__ __launch_bounds__(kSmallThreads) void k_segd_wcnt(const uint32_t *__restrict__ heads, int *wcnt,
-                                                              int64_t words, uint64_t *status, unsigned *counter,
-                                                              unsigned *err, SegdHeader *hdr, int64_t n, int64_t m,
-                                                              int pick) {
-    __shared__ unsigned s_tile;
-    __shared__ unsigned s_wave[kSmallThreads / kWave];
-    __shared__ unsigned s_total;
+// The bitmap words and head counts of one chunk.  Each head of the chunk
+// marks a byte of LDS (distinct bytes: no atomics however short the
+// segments), which the threads then pack into a word each.  With `pick`, the
+// launch has one workgroup more than chunks, and that last workgroup picks
+// the schedules from the histogram k_segd_offsets completed.
+__global__ __launch_bounds__(kChunkThreads) void k_segd_words(const int *__restrict__ offs, const int *__restrict__ nz,
+                                                             int *wcnt, uint32_t *heads, int64_t words, int64_t chunks,
+                                                             SegdHeader *hdr, int64_t n, int64_t m, int pick) {
+    constexpr int W = kChunkWords / kWave;
+    __shared__ __attribute__((aligned(16))) unsigned char s_mark[kChunk];
+    __shared__ unsigned s_wave[W];
     __shared__ unsigned s_pick[4];
-    const int tid = threadIdx.x;
-    if (pick && blockIdx.x == gridDim.x - 1) {
-        sched_pick_block(hdr, n, m, hdr->hist, s_pick);
+    const int tid = threadIdx.x, w = tid / kWave, lane = tid % kWave;
+    const int64_t c = blockIdx.x;
+    if (c == chunks) {
+        sched_pick_block<kChunkThreads>(hdr, n, m, hdr->hist, s_pick);
         return;
     }
-    const int64_t ntiles = (int64_t)gridDim.x - (pick ? 1 : 0);
-    if (tid == 0) s_tile = atomicAdd(counter, 1u);
+    const int64_t w0 = c * kChunkWords, next = w0 + kChunkWords;
+    const int all = wcnt[words];
+    int r0 = n > 0 ? wcnt[w0] : 0, r1 = next < words ? wcnt[next] : all;
+    // (lengths that do not sum to n leave some of these unwritten: clamp)
+    r0 = r0 < 0 ? 0 : (r0 > all ? all : r0);
+    r1 = r1 > all ? all : r1;
+    for (int i = tid; i < kChunk / 16; i += kChunkThreads) ((u32x4 *)s_mark)[i] = u32x4{0u, 0u, 0u, 0u};
     __syncthreads();
-    const int64_t tile = s_tile;
-    const int64_t w0 = tile * kSmallSegd + (int64_t)tid * kSmallPer;
-    unsigned loc[kSmallPer], sum = 0;
+    const int64_t lo = c * kChunk;
+    const bool ident = all == m;                  // no empty segment: nz is the identity
+#pragma unroll 8
+    for (int r = r0 + tid; r < r1; r += kChunkThreads) {
+        const int64_t o = offs[ident ? r : nz[r]];
+        if (o >= lo && o < lo + kChunk && o < n) s_mark[o - lo] = 1;
+    }
+    __syncthreads();
+    uint32_t h = 0;
+    if (tid < kChunkWords)
 #pragma unroll
-    for (int k = 0; k < kSmallPer; k++) {
-        const int64_t wd = w0 + k;
-        loc[k] = sum;
-        sum += wd < words ? (unsigned)__popc(heads[wd]) : 0u;
+    for (int q = 0; q < 2; q++) {
+        const u32x4 v = ((const u32x4 *)s_mark)[tid * 2 + q];
+        // four 0/1 bytes to four bits: the top nibble of a product that
+        // adds each byte once, shifted to its bit
+        h |= (((v.x * 0x10204080u) >> 28) | ((v.y * 0x10204080u) >> 28 << 4) | ((v.z * 0x10204080u) >> 28 << 8) |
+              ((v.w * 0x10204080u) >> 28 << 12)) << (16 * q);
     }
-    unsigned excl;
-    const unsigned P = block_tile_prefix<AddUs>(sum, s_wave, &s_total, status, tile, err, &excl);
+    const unsigned cnt = (unsigned)__popc(h);
+    const unsigned inc = wave_inclusive_scan(cnt, AddU());
+    if (w < W && lane == kWave - 1) s_wave[w] = inc;
+    __syncthreads();
+    if (tid >= kChunkWords) return;
+    unsigned base = (unsigned)r0 + inc - cnt;
 #pragma unroll
-    for (int k = 0; k < kSmallPer; k++) {
-        const int64_t wd = w0 + k;
-        if (wd < words) wcnt[wd] = (int)(P + loc[k]);
+    for (int i = 0; i < W; i++)
+        if (i < w) base += s_wave[i];
+    if (w0 + tid < words) {
+        heads[w0 + tid] = h;
+        if (tid > 0) wcnt[w0 + tid] = (int)base;
     }
-    if (tile == ntiles - 1 && tid == 0) wcnt[words] = (int)s_total;
+    if (c == chunks - 1 && tid < 8) heads[words + tid] = 0u;
 }
 
-__global__ void k_segd_empty(SegdHeader *hdr, int *offs, int64_t n) {
-    if (threadIdx.x == 0) {
-        hdr->n = n;
-        hdr->m = 0;
-        hdr->stats = kStatsMagic;
-        offs[0] = 0;
-    }
-}
-
-static int grid_cap(int64_t n, int cap = 8192) {
-    int g = grid_for(n, kBlock);
-    return g > cap ? cap : g;
-}
-
+// 16 bytes per kSmallSegd lengths hold the tile sums.
 int64_t segd_build_scratch_bytes(int64_t n, int64_t m) {
     SegdLayout L(n, m);
     const int64_t ta = (m + kSmallSegd - 1) / kSmallSegd, tb = (L.words + kSmallSegd - 1) / kSmallSegd;
+    static_assert(2 * kTile >= kSmallSegd, "the sums fit");
     return 256 + 16 * (ta + 1) + 16 * (tb + 1) + 256;
 }
 
@@ -402,29 +492,25 @@ void segd_build(void *sd, const void *lens_in, int64_t n, int64_t m, void *scrat
         LAUNCHCHECK();
         return;
     }
-    const int64_t ta = (m + kSmallSegd - 1) / kSmallSegd, tb = (L.words + kSmallSegd - 1) / kSmallSegd;
-    unsigned *counters = (unsigned *)scratch;                          // [0] pass 1, [1] pass 2
-    uint64_t *st_a = (uint64_t *)((char *)scratch + 256);
-    uint64_t *st_b = st_a + 2 * (ta + 1);
-    // scratch counters and status, the bitmap, and the header from its
-    // schedule word to the end of the histogram, in one launch
-    zero3_u32(scratch, (256 + 16 * (ta + 1) + 16 * (tb + 1)) / 4, heads, L.words + 8, &hdr->sched,
-              (int64_t)(sizeof(SegdHeader) - offsetof(SegdHeader, sched)) / 4);
-    if (m > 0) {
-        k_segd_offsets<<<(unsigned)ta, kSmallThreads, 0, g_stream>>>((const int *)lens_in, hdr, lens, offs, nz, heads,
-                                                                     n, m, st_a, counters, device_error_word());
-        LAUNCHCHECK();
-    } else {                                       // no segments: the header and offs[0] = 0
-        k_segd_empty<<<1, 64, 0, g_stream>>>(hdr, offs, n);
+    const int64_t tiles = (m + kTile - 1) / kTile;
+    const int64_t chunks = L.words > 0 ? (L.words + kChunkWords - 1) / kChunkWords : 1;
+    uint64_t *parts = (uint64_t *)((char *)scratch + 256);
+    if (tiles > 1) {
+        k_segd_sums<<<(unsigned)tiles, kTileThreads, 0, g_stream>>>((const int *)lens_in, m, parts, hdr);
         LAUNCHCHECK();
     }
-    if (L.words > 0) {
-        k_segd_wcnt<<<(unsigned)(tb + (pick ? 1 : 0)), kSmallThreads, 0, g_stream>>>(
-            heads, wcnt, L.words, st_b, counters + 1, device_error_word(), hdr, n, m, pick);
+    const int scanned = tiles > kDirectTiles;
+    if (scanned) {
+        k_segd_scan_sums<<<1, kSmallThreads, 0, g_stream>>>(parts, tiles);
         LAUNCHCHECK();
-    } else {
-        fill_u32(wcnt, 0, 1);
     }
+    // (at least one tile, so that the header of a descriptor without segments is written)
+    k_segd_offsets<<<(unsigned)(tiles > 0 ? tiles : 1), kTileThreads, 0, g_stream>>>(
+        (const int *)lens_in, hdr, lens, offs, nz, wcnt, parts, scanned, n, m);
+    LAUNCHCHECK();
+    k_segd_words<<<(unsigned)(chunks + (pick ? 1 : 0)), kChunkThreads, 0, g_stream>>>(offs, nz, wcnt, heads, L.words, chunks,
+                                                                                  hdr, n, m, pick);
+    LAUNCHCHECK();
 }
 
 }  // namespace cvlhip

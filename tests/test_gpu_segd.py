@@ -1,7 +1,7 @@
 """Segment descriptors (mke_fov) read back section by section and compared
 with their definition, for both construction paths: one workgroup for small
-descriptors (m and the bitmap's word count at most 4096), the two look-back
-kernels otherwise.
+descriptors (m and the bitmap's word count at most 4096), three kernels
+otherwise (tile sums, offsets, bitmap words).
 
 Layout (byte offsets, each section 256-byte aligned): header (n, m as
 int64) at 0; lens[m] at 256; offs[m+1] (exclusive sums, offs[m] = n); nz
@@ -57,7 +57,7 @@ def shapes():
     return [
         ("small", split(5000, 100, 0.1)),
         ("small_edge", split(4096 * 32, 4096, 0.1)),     # the largest one-workgroup descriptor
-        ("few_long", split(500_000, 3000, 0.05)),        # look-back kernels: bitmap above 4096 words
+        ("few_long", split(500_000, 3000, 0.05)),        # one tile of lengths, bitmap above 4096 words
         ("mid_tiles", split(700_000, 20_000, 0.2)),      # several tiles of lengths and of words, empties
         ("mid_edge", split(1 << 20, 1 << 15, 0.1)),      # 8 tiles of each, exactly
         ("many_short", split(120_000, 50_000, 0.2)),     # more than 4096 lengths
@@ -93,3 +93,45 @@ def test_descriptor_sections(cv, name, lens):
 def cv():
     from neslgpu_amd.cvl import Cvl
     return Cvl()
+
+
+# The three-kernel build at the edges of its tiles (2048 lengths) and chunks
+# (256 bitmap words, 8192 elements), with segments that span many chunks (a
+# wave writes their head counts together), and enough tiles that their sums
+# are scanned by a kernel of their own (above 2048 tiles).
+def edge_shapes():
+    rng = np.random.default_rng(5)
+    long = np.array([0, 40_000, 1, 0, 8192, 8191, 1, 300_000, 0, 2_000_000, 3, 0], np.int32)
+    return [("one_tile", np.full(2048, 100, np.int32)), ("tile_and_one", np.full(2049, 100, np.int32)),
+            ("long", long), ("one_long", np.array([0, 9_000_000, 0], np.int32)),
+            ("chunk_heads", np.full(300, 8192, np.int32)), ("chunk_ragged", np.full(301, 8191, np.int32)),
+            ("long_many", np.concatenate([np.ones(5000, np.int32), long, np.ones(5000, np.int32)])),
+            ("many_tiles", rng.integers(0, 3, 2048 * 2048 + 17).astype(np.int32))]
+
+
+@pytest.mark.parametrize("name,lens", edge_shapes(), ids=[s[0] for s in edge_shapes()])
+def test_descriptor_edges(cv, name, lens):
+    print("segd edge", name, lens.size, flush=True)
+    lens64 = lens.astype(np.int64)
+    n, m = int(lens64.sum()), lens.size
+    offs = np.concatenate([[0], np.cumsum(lens64)])
+    nz = np.nonzero(lens > 0)[0]
+    W, o_lens, o_offs, o_nz, o_wcnt, o_heads = layout(n, m)
+    bits = np.zeros((W + 8) * 32, np.uint8)
+    bits[offs[:-1][lens > 0]] = 1
+    heads = np.packbits(bits, bitorder="little").view(np.uint32)
+    wcnt = np.concatenate([[0], np.cumsum(bits[:W * 32].reshape(W, 32).sum(1, dtype=np.int64))])
+    raw = host(cv.segd(lens).buf).view(np.uint8)
+    i32 = lambda off, k: raw[off:off + 4 * k].view(np.int32)
+    assert list(raw[:16].view(np.int64)) == [n, m]
+    assert np.array_equal(i32(o_lens, m), lens)
+    assert np.array_equal(i32(o_offs, m + 1), offs)
+    assert np.array_equal(i32(o_nz, nz.size), nz)
+    assert np.array_equal(i32(o_wcnt, W + 1), wcnt)
+    assert np.array_equal(raw[o_heads:o_heads + 4 * (W + 8)].view(np.uint32), heads)
+    # the length-class histogram (elements, then segments, of class 2^c..2^(c+1))
+    cls = np.minimum(np.log2(lens64[nz]).astype(int), 20)
+    hist = raw[24:24 + 4 * 42].view(np.uint32)
+    assert np.array_equal(hist[:21], np.bincount(cls, lens64[nz], 21)[:21])
+    assert np.array_equal(hist[21:], np.bincount(cls, minlength=21))
+    assert cv.lib.cvlhip_check_device_errors() == 0

@@ -24,6 +24,8 @@ void cvlhip_set_error_mode(int fatal_on_error);
 /* Returns 0 if no error since the last call, else a non-zero code and the
  * message in buf. */
 int cvlhip_last_error(char *buf, int len);
+/* The code it would return, readable without a call. */
+extern int cvlhip_error_pending;
 /* Non-zero when a kernel met an out-of-range permutation index since the
  * last call (the access was skipped); clears the flag. */
 unsigned cvlhip_check_device_errors(void);

@@ -15,12 +15,17 @@
 #include <string.h>
 #include <time.h>
 
+// The code cvlhip_last_error would return, for bindings that look at it after
+// every call.
+extern "C" {
+int cvlhip_error_pending = 0;
+}
+
 namespace cvlhip {
 
 hipStream_t g_stream = nullptr;
 static int g_fatal = 1;
 static char g_errbuf[512];
-static int g_err = 0;
 static unsigned *g_dev_err = nullptr;
 
 void fatal(const char *fmt, ...) {
@@ -38,13 +43,13 @@ void usage_error(const char *fmt, ...) {
     va_start(ap, fmt);
     vsnprintf(g_errbuf, sizeof g_errbuf, fmt, ap);
     va_end(ap);
-    g_err = 1;
+    cvlhip_error_pending = 1;
     if (g_fatal) fatal("%s", g_errbuf);
 }
 
 void hip_fail(hipError_t e, const char *expr, const char *file, int line) {
     snprintf(g_errbuf, sizeof g_errbuf, "%s failed: %s (%s:%d)", expr, hipGetErrorString(e), file, line);
-    g_err = 2;
+    cvlhip_error_pending = 2;
     if (g_fatal) fatal("%s", g_errbuf);
 }
 
@@ -166,12 +171,12 @@ void *cvlhip_get_stream(void) { return (void *)g_stream; }
 void cvlhip_set_error_mode(int fatal_on_error) { g_fatal = fatal_on_error; }
 
 int cvlhip_last_error(char *buf, int len) {
-    int e = g_err;
+    int e = cvlhip_error_pending;
     if (buf && len > 0) {
-        strncpy(buf, g_err ? g_errbuf : "", (size_t)len - 1);
+        strncpy(buf, e ? g_errbuf : "", (size_t)len - 1);
         buf[len - 1] = 0;
     }
-    g_err = 0;
+    cvlhip_error_pending = 0;
     return e;
 }
 

@@ -77,8 +77,35 @@ def _addr(x):
     return x
 
 
+def _wrapper(lib: "Lib", name: str, fn, argtypes):
+    """A Python function that converts its arguments for `fn`, calls it and
+    raises a recorded error.  It is generated for the prototype, one
+    expression per argument, because most of a short call's time was this
+    (4.2 us for a call of four arguments that does nothing, with a loop over
+    the argument types; 1.0 so); the error is read from the library's own
+    word instead of with a second call."""
+    args = [f"a{k}" for k in range(len(argtypes))]
+    body, conv = [], []
+    for a, t in zip(args, argtypes):
+        if t is C.c_void_p:
+            body += [f"    try: {a} = {a}.data_ptr()", f"    except AttributeError: {a} = _addr({a})"]
+            conv.append(a)
+        elif t in (C.c_double, C.c_float):
+            conv.append(f"float({a})")
+        elif t is C.c_char_p:
+            conv.append(a)
+        else:
+            conv.append(f"int({a})")
+    src = [f"def {name}({', '.join(args)}):", *body, f"    r = _fn({', '.join(conv)})",
+           f"    if _pending.value: _check({name!r})", "    return r"]
+    env = {"_addr": _addr, "_fn": fn, "_pending": lib.pending, "_check": lib.check}
+    exec("\n".join(src), env)
+    return env[name]
+
+
 class Lib:
-    """The loaded shared library; attribute access returns checked callables."""
+    """The loaded shared library; its functions are attributes, made on first
+    use."""
 
     def __init__(self, path: str = LIB_PATH):
         if not os.path.exists(path):
@@ -90,6 +117,7 @@ class Lib:
             f = getattr(self.dll, name)
             f.restype = rt
             f.argtypes = ats
+        self.pending = C.c_int.in_dll(self.dll, "cvlhip_error_pending")
         self.dll.cvlhip_set_error_mode(0)
         self._buf = C.create_string_buffer(512)
 
@@ -99,29 +127,11 @@ class Lib:
             raise CvlError(f"{name}: {self._buf.value.decode()}")
 
     def __getattr__(self, name):
+        # reached once per function: the wrapper is kept as an attribute
         if name.startswith("_") or name not in self.protos:
             raise AttributeError(name)
-        f = getattr(self.dll, name)
-        rt, ats = self.protos[name]
-
-        def call(*args):
-            if len(args) != len(ats):
-                raise TypeError(f"{name} takes {len(ats)} arguments, got {len(args)}")
-            conv = []
-            for a, t in zip(args, ats):
-                if t in (C.c_void_p,):
-                    conv.append(_addr(a))
-                elif t is C.c_double or t is C.c_float:
-                    conv.append(float(a))
-                elif t is C.c_char_p:
-                    conv.append(a)
-                else:
-                    conv.append(int(a))
-            r = f(*conv)
-            self.check(name)
-            return r
-
-        call.__name__ = name
+        call = _wrapper(self, name, getattr(self.dll, name), self.protos[name][1])
+        setattr(self, name, call)
         return call
 
 

@@ -2,8 +2,9 @@
 // replace, copies and RAND (ref nesl/cvl/serial/elwise.c:128-298,
 // vprims.c:203-344, library.c:9-49, facilt.c:292-312).
 //
-// Elementwise kernels are grid-stride loops (coalesced 4- or 8-byte lane
-// accesses); one read of each input and one write of the output.  Arithmetic follows C on the
+// An elementwise workgroup owns a tile and each lane U vectors of it (16 bytes
+// of the widest operand), all loaded before the first is used; one read of
+// each input and one write of the output.  Arithmetic follows C on the
 // host: int overflow wraps, int / and % truncate, floating point is compiled
 // without contraction (-ffp-contract=off) so + - * / and sqrt round exactly
 // as the serial CVL; libm transcendentals may differ in the last ulp.
@@ -24,29 +25,191 @@ static int ew_grid(int64_t n) {
 }
 
 // ------------------------------------------------------------------ kernels
-template <class F>
-__global__ void k_ew2(typename F::Out *__restrict__ d, const typename F::In *__restrict__ a,
-                      const typename F::In *__restrict__ b, int64_t n) {
-    const F f;
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (; i < n; i += stride) d[i] = f(a[i], b[i]);
+// V consecutive elements of one operand, as one load or store.
+template <class T, int V> struct EwVec { typedef T type __attribute__((ext_vector_type(V))); };
+
+// Elements per lane and vector: 16 bytes of the widest operand.
+template <class... T>
+constexpr int ew_lane() {
+    size_t w = 4;
+    ((w = sizeof(T) > w ? sizeof(T) : w), ...);
+    return (int)(16 / w);
 }
 
-template <class F>
-__global__ void k_ew1(typename F::Out *__restrict__ d, const typename F::In *__restrict__ a, int64_t n) {
+// Vectors per lane of a long vector; vectors so short that larger tiles would
+// leave CUs without a workgroup take one.  Bound by memory.  Nine calls of
+// quickhull's test (three of four 24 B/element) of 2^26 doubles, and five of
+// 16-byte-per-element int work: 2708 and 866 us with grid-stride loops of one
+// element per lane, 2335 and 751 with two vectors per lane (5.6 and 5.7
+// TB/s), 2322 and 758 with four, 2418 and 770 with eight; of 4 10^6 elements,
+// which the caches hold, 139 and 43, then 126 and 39, 129 and 48, 137 and 44.
+constexpr int kEwLong = 2;
+constexpr int64_t kEwLongMin = 1 << 21;
+
+// A workgroup's tile is kBlock * U * V elements, V = ew_lane; the last one,
+// and vectors that do not start on 16 bytes, go element by element.  d may be
+// one of the inputs (all of a lane's loads precede its stores).
+template <class F, int U>
+__global__ __launch_bounds__(kBlock) void k_ew2(typename F::Out *d, const typename F::In *a, const typename F::In *b,
+                                                int64_t n, int aligned) {
+    using In = typename F::In;
+    using Out = typename F::Out;
+    constexpr int V = ew_lane<In, Out>();
+    using VI = typename EwVec<In, V>::type;
+    using VO = typename EwVec<Out, V>::type;
     const F f;
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (; i < n; i += stride) d[i] = f(a[i]);
+    const int64_t t0 = (int64_t)blockIdx.x * (kBlock * U * V);
+    if (aligned && t0 + kBlock * U * V <= n) {
+        VI x[U], y[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int64_t e = t0 + (u * kBlock + (int)threadIdx.x) * V;
+            x[u] = *(const VI *)(a + e);
+            y[u] = *(const VI *)(b + e);
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            VO o;
+#pragma unroll
+            for (int k = 0; k < V; k++) o[k] = f(x[u][k], y[u][k]);
+            *(VO *)(d + t0 + (u * kBlock + (int)threadIdx.x) * V) = o;
+        }
+        return;
+    }
+    for (int64_t i = t0 + threadIdx.x; i < n && i < t0 + kBlock * U * V; i += kBlock) d[i] = f(a[i], b[i]);
 }
 
+template <class F, int U>
+__global__ __launch_bounds__(kBlock) void k_ew1(typename F::Out *d, const typename F::In *a, int64_t n, int aligned) {
+    using In = typename F::In;
+    using Out = typename F::Out;
+    constexpr int V = ew_lane<In, Out>();
+    using VI = typename EwVec<In, V>::type;
+    using VO = typename EwVec<Out, V>::type;
+    const F f;
+    const int64_t t0 = (int64_t)blockIdx.x * (kBlock * U * V);
+    if (aligned && t0 + kBlock * U * V <= n) {
+        VI x[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) x[u] = *(const VI *)(a + t0 + (u * kBlock + (int)threadIdx.x) * V);
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            VO o;
+#pragma unroll
+            for (int k = 0; k < V; k++) o[k] = f(x[u][k]);
+            *(VO *)(d + t0 + (u * kBlock + (int)threadIdx.x) * V) = o;
+        }
+        return;
+    }
+    for (int64_t i = t0 + threadIdx.x; i < n && i < t0 + kBlock * U * V; i += kBlock) d[i] = f(a[i]);
+}
+
+template <class T, int U>
+__global__ __launch_bounds__(kBlock) void k_sel(T *d, const int *f, const T *a, const T *b, int64_t n, int aligned) {
+    constexpr int V = ew_lane<T>();
+    using VF = typename EwVec<int, V>::type;
+    using VT = typename EwVec<T, V>::type;
+    const int64_t t0 = (int64_t)blockIdx.x * (kBlock * U * V);
+    if (aligned && t0 + kBlock * U * V <= n) {
+        VF g[U];
+        VT x[U], y[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int64_t e = t0 + (u * kBlock + (int)threadIdx.x) * V;
+            g[u] = *(const VF *)(f + e);
+            x[u] = *(const VT *)(a + e);
+            y[u] = *(const VT *)(b + e);
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            VT o;
+#pragma unroll
+            for (int k = 0; k < V; k++) o[k] = g[u][k] ? x[u][k] : y[u][k];
+            *(VT *)(d + t0 + (u * kBlock + (int)threadIdx.x) * V) = o;
+        }
+        return;
+    }
+    for (int64_t i = t0 + threadIdx.x; i < n && i < t0 + kBlock * U * V; i += kBlock) d[i] = f[i] ? a[i] : b[i];
+}
+
+// The value at(k) in every element k of d.
+template <class T, class F, int U>
+__global__ __launch_bounds__(kBlock) void k_make(T *d, F at, int64_t n, int aligned) {
+    constexpr int V = ew_lane<T>();
+    using VT = typename EwVec<T, V>::type;
+    const int64_t t0 = (int64_t)blockIdx.x * (kBlock * U * V);
+    if (aligned && t0 + kBlock * U * V <= n) {
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int64_t e = t0 + (u * kBlock + (int)threadIdx.x) * V;
+            VT o;
+#pragma unroll
+            for (int k = 0; k < V; k++) o[k] = at(e + k);
+            *(VT *)(d + e) = o;
+        }
+        return;
+    }
+    for (int64_t i = t0 + threadIdx.x; i < n && i < t0 + kBlock * U * V; i += kBlock) d[i] = at(i);
+}
 template <class T>
-__global__ void k_sel(T *__restrict__ d, const int *__restrict__ f, const T *__restrict__ a,
-                      const T *__restrict__ b, int64_t n) {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (; i < n; i += stride) d[i] = f[i] ? a[i] : b[i];
+struct ConstAt {
+    T v;
+    __device__ T operator()(int64_t) const { return v; }
+};
+struct StepAt {
+    int init, step;
+    __device__ int operator()(int64_t i) const { return (int)((unsigned)init + (unsigned)step * (unsigned)i); }
+};
+
+// Are all operands 16-byte aligned?
+template <class... P>
+static int ew_aligned(P... p) {
+    return (((uintptr_t)p | ...) & 15) == 0;
+}
+
+template <class F>
+static void launch_ew2(void *d, const void *a, const void *b, int64_t n) {
+    using In = typename F::In;
+    using Out = typename F::Out;
+    constexpr int T1 = kBlock * ew_lane<In, Out>();
+    const int al = ew_aligned(d, a, b);
+    if (n < kEwLongMin)
+        k_ew2<F, 1><<<grid_for(n, T1), kBlock, 0, g_stream>>>((Out *)d, (const In *)a, (const In *)b, n, al);
+    else
+        k_ew2<F, kEwLong><<<grid_for(n, T1 * kEwLong), kBlock, 0, g_stream>>>((Out *)d, (const In *)a, (const In *)b, n, al);
+    LAUNCHCHECK();
+}
+// U: vectors per lane of a long vector; 1 for functions long enough to hide
+// the loads.
+template <class F, int U>
+static void launch_ew1(void *d, const void *a, int64_t n) {
+    using In = typename F::In;
+    using Out = typename F::Out;
+    constexpr int T1 = kBlock * ew_lane<In, Out>();
+    const int al = ew_aligned(d, a);
+    if (U == 1 || n < kEwLongMin)
+        k_ew1<F, 1><<<grid_for(n, T1), kBlock, 0, g_stream>>>((Out *)d, (const In *)a, n, al);
+    else
+        k_ew1<F, U><<<grid_for(n, T1 * U), kBlock, 0, g_stream>>>((Out *)d, (const In *)a, n, al);
+    LAUNCHCHECK();
+}
+template <class T>
+static void launch_sel(void *d, const void *f, const void *a, const void *b, int64_t n) {
+    constexpr int T1 = kBlock * ew_lane<T>();
+    const int al = ew_aligned(d, f, a, b);
+    if (n < kEwLongMin)
+        k_sel<T, 1><<<grid_for(n, T1), kBlock, 0, g_stream>>>((T *)d, (const int *)f, (const T *)a, (const T *)b, n, al);
+    else
+        k_sel<T, kEwLong><<<grid_for(n, T1 * kEwLong), kBlock, 0, g_stream>>>((T *)d, (const int *)f, (const T *)a,
+                                                                              (const T *)b, n, al);
+    LAUNCHCHECK();
+}
+template <class T, class F>
+static void launch_make(void *d, F at, int64_t n) {
+    constexpr int T1 = kBlock * ew_lane<T>();
+    if (n < kEwLongMin) k_make<T, F, 1><<<grid_for(n, T1), kBlock, 0, g_stream>>>((T *)d, at, n, ew_aligned(d));
+    else k_make<T, F, kEwLong><<<grid_for(n, T1 * kEwLong), kBlock, 0, g_stream>>>((T *)d, at, n, ew_aligned(d));
+    LAUNCHCHECK();
 }
 
 // one element written by one lane (scalar replace without a host wait)
@@ -59,13 +222,6 @@ __global__ void k_put1(T *p, T v) {
 template <class T>
 __global__ void k_ext_post(const T *p, Mailbox *mb, unsigned long long seq) {
     if (threadIdx.x == 0) mailbox_post(mb, seq, scalar_bits(*p));
-}
-
-template <class T>
-__global__ void k_dist(T *__restrict__ d, T v, int64_t n) {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (; i < n; i += stride) d[i] = v;
 }
 
 template <class T>
@@ -87,12 +243,6 @@ __global__ void k_dist_seg(T *__restrict__ d, const T *__restrict__ v, SegdView 
         for (int u = 0; u < 4; u++)
             if (i + u * stride < sv.n) d[i + u * stride] = x[u];
     }
-}
-
-__global__ void k_index(int *__restrict__ d, int init, int stride_v, int64_t n) {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (; i < n; i += stride) d[i] = (int)((unsigned)init + (unsigned)stride_v * (unsigned)i);
 }
 
 __global__ void k_index_seg(int *__restrict__ d, const int *__restrict__ init, const int *__restrict__ st,
@@ -210,18 +360,16 @@ using namespace cvlhip;
     void NAME(vec_p d, vec_p s1, vec_p s2, int len, vec_p scratch) {                          \
         (void)scratch;                                                                        \
         if (len <= 0) return;                                                                 \
-        k_ew2<F><<<ew_grid(len), kBlock, 0, g_stream>>>((F::Out *)d, (const F::In *)s1,       \
-                                                        (const F::In *)s2, len);              \
-        LAUNCHCHECK();                                                                        \
+        launch_ew2<F>(d, s1, s2, len);                                                        \
     }                                                                                         \
     NOSCR(NAME, FLAG)
 
-#define EW1(NAME, F, FLAG)                                                                    \
+#define EW1(NAME, F, FLAG) EW1U(NAME, F, FLAG, kEwLong)
+#define EW1U(NAME, F, FLAG, U)                                                                 \
     void NAME(vec_p d, vec_p s, int len, vec_p scratch) {                                     \
         (void)scratch;                                                                        \
         if (len <= 0) return;                                                                 \
-        k_ew1<F><<<ew_grid(len), kBlock, 0, g_stream>>>((F::Out *)d, (const F::In *)s, len);  \
-        LAUNCHCHECK();                                                                        \
+        launch_ew1<F, U>(d, s, len);                                                          \
     }                                                                                         \
     NOSCR(NAME, FLAG)
 
@@ -263,18 +411,18 @@ EW1(flr_wud, FlrDf, INPLACE_NONE)
 EW1(cei_wud, CeiDf, INPLACE_NONE)
 EW1(trn_wud, TrnDf, INPLACE_NONE)
 EW1(rou_wud, RouDf, INPLACE_NONE)
-EW1(exp_wud, ExpDf, INPLACE_1)
-EW1(log_wud, LogDf, INPLACE_1)
+EW1U(exp_wud, ExpDf, INPLACE_1, 1)
+EW1U(log_wud, LogDf, INPLACE_1, 1)
 EW1(sqt_wud, SqtDf, INPLACE_1)
-EW1(sin_wud, SinDf, INPLACE_1)
-EW1(cos_wud, CosDf, INPLACE_1)
-EW1(tan_wud, TanDf, INPLACE_1)
-EW1(asn_wud, AsnDf, INPLACE_1)
-EW1(acs_wud, AcsDf, INPLACE_1)
-EW1(atn_wud, AtnDf, INPLACE_1)
-EW1(snh_wud, SnhDf, INPLACE_1)
-EW1(csh_wud, CshDf, INPLACE_1)
-EW1(tnh_wud, TnhDf, INPLACE_1)
+EW1U(sin_wud, SinDf, INPLACE_1, 1)
+EW1U(cos_wud, CosDf, INPLACE_1, 1)
+EW1U(tan_wud, TanDf, INPLACE_1, 1)
+EW1U(asn_wud, AsnDf, INPLACE_1, 1)
+EW1U(acs_wud, AcsDf, INPLACE_1, 1)
+EW1U(atn_wud, AtnDf, INPLACE_1, 1)
+EW1U(snh_wud, SnhDf, INPLACE_1, 1)
+EW1U(csh_wud, CshDf, INPLACE_1, 1)
+EW1U(tnh_wud, TnhDf, INPLACE_1, 1)
 
 #define CPY(NAME, W)                                                                           \
     void NAME(vec_p d, vec_p s, int len, vec_p scratch) {                                      \
@@ -291,8 +439,7 @@ CPY(cpy_wud, 8)
     void NAME(vec_p d, vec_p s1, vec_p s2, vec_p s3, int len, vec_p scratch) {                 \
         (void)scratch;                                                                         \
         if (len <= 0) return;                                                                  \
-        k_sel<T><<<ew_grid(len), kBlock, 0, g_stream>>>((T *)d, (const int *)s1, (const T *)s2, (const T *)s3, len); \
-        LAUNCHCHECK();                                                                         \
+        launch_sel<T>(d, s1, s2, s3, len);                                                     \
     }                                                                                          \
     NOSCR(NAME, INPLACE_1 | INPLACE_2 | INPLACE_3)
 SEL(sel_wuz, int)
@@ -323,8 +470,7 @@ unsigned long long cvlhip_rand_get_state(void) { return g_rand_state; }
     void NAME(vec_p d, T v, int len, vec_p scratch) {                                          \
         (void)scratch;                                                                         \
         if (len <= 0) return;                                                                  \
-        k_dist<T><<<ew_grid(len), kBlock, 0, g_stream>>>((T *)d, v, len);                      \
-        LAUNCHCHECK();                                                                         \
+        launch_make<T>(d, ConstAt<T>{v}, len);                                                 \
     }                                                                                          \
     NOSCR(NAME, INPLACE_NONE)
 DIS(dis_vuz, int)
@@ -332,8 +478,7 @@ DIS(dis_vud, double)
 void dis_vub(vec_p d, cvl_bool v, int len, vec_p scratch) {
     (void)scratch;
     if (len <= 0) return;
-    k_dist<int><<<ew_grid(len), kBlock, 0, g_stream>>>((int *)d, v, len);
-    LAUNCHCHECK();
+    launch_make<int>(d, ConstAt<int>{v}, len);
 }
 NOSCR(dis_vub, INPLACE_NONE)
 
@@ -354,8 +499,7 @@ DISSEG(dis_ved, double, dis_vud)
 void ind_luz(vec_p d, int init, int stride, int count, vec_p scratch) {
     (void)scratch;
     if (count <= 0) return;
-    k_index<<<ew_grid(count), kBlock, 0, g_stream>>>((int *)d, init, stride, count);
-    LAUNCHCHECK();
+    launch_make<int>(d, StepAt{init, stride}, count);
 }
 NOSCR(ind_luz, INPLACE_NONE)
 

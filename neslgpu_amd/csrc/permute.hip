@@ -67,6 +67,54 @@ __global__ void k_gather(T *__restrict__ d, const T *__restrict__ s, const int *
     }
 }
 
+// The plain gather, d[k] = s[i[k]] for every k: four elements per lane, their
+// loads of s in flight together.  Bound by the random loads of s, about 60 G/s
+// once s exceeds an XCD's L2.  STREAM (long vectors): the indices and the
+// result pass by the caches, which are left to s.  An SpMV product of 2^26
+// nonzeros whose x holds 2^22 / 2^20 doubles: 1614 / 1158 us with one element
+// per lane, 1609 / 1139 with four, 1600 / 1097 streamed (of 3 10^6 nonzeros
+// all the same; non-temporal loads of x: 1931 / 1603).
+constexpr int kGatherTile = kBlock * 4;
+constexpr int64_t kGatherStreamMin = 1 << 22;
+template <class T, bool STREAM>
+__global__ __launch_bounds__(kBlock) void k_gather_flat(T *d, const T *__restrict__ s, const int *idx, int64_t n_d,
+                                                        int64_t n_s, int aligned, unsigned *err) {
+    typedef int i32x4 __attribute__((ext_vector_type(4)));
+    constexpr int E = 16 / (int)sizeof(T);
+    typedef T vt __attribute__((ext_vector_type(E)));
+    const int64_t t0 = (int64_t)blockIdx.x * kGatherTile;
+    if (aligned && t0 + kGatherTile <= n_d) {
+        const i32x4 *const p = (const i32x4 *)(idx + t0) + threadIdx.x;
+        const i32x4 q = STREAM ? __builtin_nontemporal_load(p) : *p;
+        T v[4];
+        bool bad = false;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const int i = q[k];
+            const bool in = i >= 0 && i < n_s;
+            bad |= !in;
+            const T x = s[in ? i : 0];
+            v[k] = in ? x : T(0);
+        }
+        vt *const o = (vt *)(d + t0) + threadIdx.x * (4 / E);
+#pragma unroll
+        for (int h = 0; h < 4 / E; h++) {
+            vt w;
+#pragma unroll
+            for (int k = 0; k < E; k++) w[k] = v[h * E + k];
+            if (STREAM) __builtin_nontemporal_store(w, o + h);
+            else o[h] = w;
+        }
+        if (bad) *err = 1u;
+        return;
+    }
+    for (int64_t k = t0 + threadIdx.x; k < n_d && k < t0 + kGatherTile; k += kBlock) {
+        const int64_t i = idx[k];
+        if (i >= 0 && i < n_s) d[k] = s[i];
+        else { d[k] = T(0); *err = 1u; }
+    }
+}
+
 // Last-writer-wins scatter, pass 1: win[p] = max source position aimed at p.
 __global__ void k_claim(int *__restrict__ win, const int *__restrict__ idx, const int *__restrict__ f, int64_t n,
                         int64_t n_d, SegBase sb) {
@@ -108,6 +156,18 @@ void scatter(void *d, const void *s, const void *idx, const void *f, int64_t n, 
 template <class T>
 void gather(void *d, const void *s, const void *idx, const void *f, int64_t n_d, int64_t n_s, SegBase sb) {
     if (n_d <= 0) return;
+    if (!f && !sb.seg && n_s > 0) {        // (with nothing to gather from, every index is out of range)
+        const int aligned = (((uintptr_t)d | (uintptr_t)idx) & 15) == 0;
+        const unsigned g = (unsigned)grid_for(n_d, kGatherTile);
+        if (n_d >= kGatherStreamMin)
+            k_gather_flat<T, true><<<g, kBlock, 0, g_stream>>>((T *)d, (const T *)s, (const int *)idx, n_d, n_s, aligned,
+                                                              device_error_word());
+        else
+            k_gather_flat<T, false><<<g, kBlock, 0, g_stream>>>((T *)d, (const T *)s, (const int *)idx, n_d, n_s, aligned,
+                                                               device_error_word());
+        LAUNCHCHECK();
+        return;
+    }
     k_gather<T><<<pgrid(n_d), kBlock, 0, g_stream>>>((T *)d, (const T *)s, (const int *)idx, (const int *)f, n_d,
                                                      n_s, sb, device_error_word());
     LAUNCHCHECK();

@@ -310,6 +310,22 @@ Mailbox *mailbox_device();                              // device address (alloc
 unsigned long long mailbox_next();                      // sequence number of the next post
 unsigned long long mailbox_wait(unsigned long long seq);   // host: the value posted with seq
 
+// Where the blocks of a reduction that the host waits for leave their
+// partials: counters that return to 0 with each call, and for each of up to
+// kReducePartials blocks one word per 32 bits of its partial, under the low
+// half of the call's sequence number.  The library's own memory, so that a
+// word carries a number only if that call wrote it; calls that wait for the
+// host never overlap.  Cleared whenever the low half wraps (mailbox_next).
+constexpr int kReducePartials = 2048;
+constexpr int kShareGroups = 32;
+struct ReduceShare {
+    struct {
+        unsigned n, pad[31];                // a cache line each
+    } count[1 + kShareGroups];
+    uint64_t words[2 * kReducePartials];
+};
+ReduceShare *reduce_share();                            // device address (allocated with the mailbox)
+
 __device__ __forceinline__ void mailbox_post(Mailbox *mb, unsigned long long seq, unsigned long long bits) {
     __hip_atomic_store(&mb->value, bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     __hip_atomic_store(&mb->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);

@@ -75,6 +75,7 @@ __global__ void k_fill_u32(uint32_t *__restrict__ p, uint32_t v, int64_t count) 
 static Mailbox *g_mb_host = nullptr;
 static Mailbox *g_mb_dev = nullptr;
 static unsigned long long g_mb_seq = 0;
+static ReduceShare *g_share = nullptr;
 
 Mailbox *mailbox_device() {
     if (!g_mb_host) {
@@ -83,11 +84,22 @@ Mailbox *mailbox_device() {
         g_mb_host->seq = 0;
         g_mb_host->value = 0;
         HIPCHECK(hipHostGetDevicePointer((void **)&g_mb_dev, g_mb_host, 0));
+        // synchronous clear, before any kernel can read it
+        HIPCHECK(hipMalloc((void **)&g_share, sizeof(ReduceShare)));
+        HIPCHECK(hipMemset(g_share, 0, sizeof(ReduceShare)));
     }
     return g_mb_dev;
 }
 
-unsigned long long mailbox_next() { return ++g_mb_seq; }
+ReduceShare *reduce_share() { return g_share; }
+
+unsigned long long mailbox_next() {
+    if ((uint32_t)++g_mb_seq == 0) {       // the words' numbers wrap: forget the old ones
+        ++g_mb_seq;
+        if (g_share) fill_u32(g_share, 0, sizeof(ReduceShare) / 4);
+    }
+    return g_mb_seq;
+}
 
 // Spins on the sequence number for up to 2 ms, then waits for the stream
 // (which reports a failed kernel) and looks once more.

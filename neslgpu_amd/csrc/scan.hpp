@@ -21,7 +21,6 @@ int64_t seg_reduce_scratch_bytes(int64_t n, int elem_bytes);
 
 // Scratch of an unsegmented reduction: a 256-byte header, one 8-byte slot
 // per block partial, and the result slot (at kReduceResultOffset).
-constexpr int kReducePartials = 2048;     // most blocks of one reduction
 constexpr int64_t kReduceResultOffset = 256 + (int64_t)kReducePartials * 8;
 constexpr int64_t kReduceScratchBytes = kReduceResultOffset + 256;
 

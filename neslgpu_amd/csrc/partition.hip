@@ -29,7 +29,6 @@
 #include "segd.hpp"
 #include "partition.hpp"
 #include "colscan.hpp"
-#include "lookback.hpp"
 #include "../../include/cvl.h"
 
 namespace cvlhip {
@@ -52,20 +51,6 @@ constexpr int blk_log() { return sizeof(T) == 4 ? kBlkLog4 : kBlkLog8; }
 #ifndef CVLHIP_PART_THREADS
 #define CVLHIP_PART_THREADS 1024
 #endif
-// 1: the first pass chains each tile's slots in the children from the tiles
-// before it (look-back) instead of a histogram pass over the indices and a
-// column scan.
-#ifndef CVLHIP_PART_LOOKBACK
-#define CVLHIP_PART_LOOKBACK 0
-#endif
-constexpr bool kPartLookback = CVLHIP_PART_LOOKBACK != 0;
-// 1: the first pass claims its slots like the later passes, one atomic per
-// (tile, child), instead of a histogram pass over the indices and a
-// column scan.
-#ifndef CVLHIP_PART_ATOMIC_FIRST
-#define CVLHIP_PART_ATOMIC_FIRST 0
-#endif
-constexpr bool kPartAtomicFirst = CVLHIP_PART_ATOMIC_FIRST != 0 && !kPartLookback;
 constexpr int kPartThreads = CVLHIP_PART_THREADS;
 constexpr int kPartItems = CVLHIP_PART_ITEMS;
 constexpr int kPartTile = kPartThreads * kPartItems;   // pairs per tile
@@ -203,17 +188,33 @@ struct Local16 {
     }
 };
 
+// Do all active lanes hold the same d?
+__device__ __forceinline__ bool wave_same(int d) {
+    return ballot(d == __builtin_amdgcn_readfirstlane(d)) == ballot(true);
+}
+// The place of this lane's element among those of bucket d so far, counted in
+// LDS.  `runs`: the wave's elements may well all aim at one bucket
+// (neighbours of a rotation or another order that keeps runs together); they
+// then count themselves with one atomic instead of 64 that take turns: a
+// rotation of 2^26 ints 1040 -> 582 us, a random order 597 -> 587.
+__device__ __forceinline__ unsigned bucket_place(unsigned *hist, int d, bool runs) {
+    if (!runs || !wave_same(d)) return atomicAdd(&hist[d], 1u);
+    const uint64_t all = ballot(true);
+    const unsigned before = __builtin_amdgcn_mbcnt_hi((uint32_t)(all >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)all, 0u));
+    unsigned at = 0;
+    if (before == 0) at = atomicAdd(&hist[d], (unsigned)__popcll(all));
+    return (unsigned)__builtin_amdgcn_readfirstlane((int)at) + before;
+}
+
 // One partition pass.  Region r = [r*psize, min((r+1)*psize, n)) of the
 // input is split into children of csize elements (csize divides psize,
 // psize/csize <= 256).  Block b handles tile (b % tiles_per_region) of
 // region (b / tiles_per_region).  Child c's pairs land in
 // [c*csize, c*csize + cnt[c]) of the output.
-// A first pass takes each tile's slot in each child from tile_ofs (the
-// column scan of per-tile histograms) or, with `lb`, from a look-back over
-// the tiles before it: tiles are then claimed in order from lb_ctr, every
-// tile publishes its counts and adds up the earlier ones child by child
-// (a tile waits only on tiles already claimed, so every wait ends), and the
-// last tile writes the children's totals to cnt.
+// Each tile's slot in each child comes from tile_ofs (the column scan of
+// per-tile histograms: long first passes) or is claimed with one atomic per
+// non-empty child.  cstride, pstride: words from one child's counter to the
+// next, in cnt and prev_cnt.
 template <class T, bool FIRST, class Out = Pairs<T>>
 __global__ __launch_bounds__(kPartThreads) void k_partition(IndexSource src, Pairs<T> in,
                                                             const T *__restrict__ in_val, Out out,
@@ -222,13 +223,11 @@ __global__ __launch_bounds__(kPartThreads) void k_partition(IndexSource src, Pai
                                                             const unsigned *__restrict__ prev_cnt,
                                                             unsigned *__restrict__ cnt,
                                                             const unsigned *__restrict__ tile_ofs,
-                                                            unsigned *__restrict__ err,
-                                                            uint32_t *__restrict__ lb = nullptr,
-                                                            unsigned *__restrict__ lb_ctr = nullptr) {
+                                                            int cstride, int pstride,
+                                                            unsigned *__restrict__ err) {
     __shared__ unsigned s_hist[kMaxFan];
     __shared__ unsigned s_start[kMaxFan];
     __shared__ unsigned s_gofs[kMaxFan];
-    __shared__ unsigned s_bt;
     // The tile staged in bucket order: four-byte values share one 8-byte
     // word with their index (one LDS access each way, and the bucket is
     // recomputed from the index); wider values keep the index, the value
@@ -240,16 +239,14 @@ __global__ __launch_bounds__(kPartThreads) void k_partition(IndexSource src, Pai
     __shared__ unsigned char s_dig[PACKED ? 1 : kPartTile];
 
     const int tid = threadIdx.x;
-    constexpr bool LB = FIRST && kPartLookback;    // compiled in only when selected
     for (int i = tid; i < kMaxFan; i += kPartThreads) s_hist[i] = 0;
-    if (LB && tid == 0) s_bt = atomicAdd(lb_ctr, 1u);
     __syncthreads();
-    const int64_t bt = LB ? (int64_t)s_bt : xcd_tile(blockIdx.x, gridDim.x);
+    const int64_t bt = xcd_tile(blockIdx.x, gridDim.x);
     const int64_t region = bt / tiles_per_region;
     const int64_t chunk = bt % tiles_per_region;
     const int64_t rlo = region << plog;
     int64_t rhi = (rlo + ((int64_t)1 << plog)) < n ? rlo + ((int64_t)1 << plog) : n;
-    if (!FIRST && rlo + (int64_t)prev_cnt[region] < rhi) rhi = rlo + prev_cnt[region];   // pairs that landed
+    if (!FIRST && rlo + (int64_t)prev_cnt[region * pstride] < rhi) rhi = rlo + prev_cnt[region * pstride];   // pairs that landed
     const int64_t lo = rlo + chunk * kPartTile;
     const int64_t first_child = rlo >> clog;
 
@@ -302,9 +299,15 @@ __global__ __launch_bounds__(kPartThreads) void k_partition(IndexSource src, Pai
             }
         }
     }
+    // whether a lane's runs of kPartV elements lie in one bucket with the
+    // other lanes' is tried on the first of each run (4-byte values only: the
+    // passes of wider ones, with fewer waves in flight, lose 1.5% by it on
+    // random orders)
+    bool runs = false;
 #pragma unroll
     for (int j = 0; j < kPartItems; j++) {
         dg[j] = -1;
+        if (PACKED && j % kPartV == 0) runs = wave_same((int)(qv[j] >> clog));
         if (has[j]) {
             const int64_t qq = qv[j];
             const int64_t child = qq >> clog;
@@ -312,7 +315,7 @@ __global__ __launch_bounds__(kPartThreads) void k_partition(IndexSource src, Pai
             if (qq >= 0 && qq < n && d >= 0 && d < kMaxFan && (qq >> plog) == region) {
                 q[j] = (int)qq;
                 dg[j] = (int)d;
-                rk[j] = atomicAdd(&s_hist[d], 1u);
+                rk[j] = bucket_place(s_hist, (int)d, runs);
             } else {
                 atomicOr(err, 1u);
             }
@@ -335,22 +338,14 @@ __global__ __launch_bounds__(kPartThreads) void k_partition(IndexSource src, Pai
             run += c[i];
         }
     }
-    if (!LB && tid < kMaxFan) {
+    if (tid < kMaxFan) {
         const int d = tid;
         if (tile_ofs) {
             s_gofs[d] = tile_ofs[bt * kMaxFan + d];
         } else {
             const unsigned c = s_hist[d];
-            s_gofs[d] = c ? atomicAdd(cnt + first_child + d, c) : 0u;
+            s_gofs[d] = c ? atomicAdd(cnt + (first_child + d) * cstride, c) : 0u;
         }
-    }
-    if (LB && tid < kMaxFan) {
-        // one thread per child: the counts of the tiles before this one
-        const int d = tid;
-        const unsigned c = s_hist[d];
-        const unsigned excl = chain_exclusive(lb, bt, kMaxFan, d, c, 0, err);
-        s_gofs[d] = excl;
-        if (bt == (int64_t)gridDim.x - 1) cnt[first_child + d] = excl + c;
     }
     __syncthreads();
 #pragma unroll
@@ -420,9 +415,10 @@ __global__ __launch_bounds__(kPartThreads) void k_part_hist(IndexSource src, int
 #pragma unroll
         for (int g = 0; g < kPartItems / kPartV; g++) {
             const unsigned q[4] = {w[g].x, w[g].y, w[g].z, w[g].w};
+            const bool runs = wave_same((int)(q[0] >> clog));
 #pragma unroll
             for (int c = 0; c < 4; c++)
-                if (q[c] < (uint64_t)n) atomicAdd(&s_hist[q[c] >> clog], 1u);
+                if (q[c] < (uint64_t)n) bucket_place(s_hist, (int)(q[c] >> clog), runs);
         }
         __syncthreads();
         for (int d = tid; d < kMaxFan; d += kPartThreads) hist[bt * kMaxFan + d] = s_hist[d];
@@ -461,12 +457,12 @@ __global__ __launch_bounds__(kPartThreads) void k_block_scatter(IndexSource src,
                                                                 unsigned *__restrict__ err) {
     constexpr int64_t kBlk = (int64_t)1 << blk_log<T>();
     __shared__ T s_out[kBlk];
-    __shared__ unsigned s_mask[kBlk / 32];
+    __shared__ __attribute__((aligned(16))) unsigned char s_mark[kBlk];   // written (bytes: no two lanes share one)
     const int tid = threadIdx.x;
     const int64_t blk = xcd_tile(blockIdx.x, gridDim.x);
     const int64_t base = blk * kBlk;
     const int64_t end = base + kBlk < n ? base + kBlk : n;
-    for (int i = tid; i < kBlk / 32; i += kPartThreads) s_mask[i] = 0;
+    for (int i = tid; i < kBlk / 16; i += kPartThreads) ((u32x4 *)s_mark)[i] = u32x4{0u, 0u, 0u, 0u};
     __syncthreads();
     int64_t count = end - base;
     if (!DIRECT && (int64_t)cnt[blk] < count) count = cnt[blk];
@@ -474,7 +470,7 @@ __global__ __launch_bounds__(kPartThreads) void k_block_scatter(IndexSource src,
         const int64_t o = In::LOCAL ? (q & (kBlk - 1)) : q - base;
         if (o >= 0 && o < end - base) {
             s_out[o] = v;
-            atomicOr(&s_mask[o >> 5], 1u << (o & 31));
+            s_mark[o] = 1;
         } else {
             atomicOr(err, 1u);
         }
@@ -500,7 +496,7 @@ __global__ __launch_bounds__(kPartThreads) void k_block_scatter(IndexSource src,
     }
     __syncthreads();
     for (int64_t o = tid; o < end - base; o += kPartThreads)
-        if ((s_mask[o >> 5] >> (o & 31)) & 1u) d[base + o] = s_out[o];
+        if (s_mark[o]) d[base + o] = s_out[o];
 }
 
 // Direct permute of vectors that stay in the caches: every value is stored
@@ -589,6 +585,19 @@ static void launch_permute_direct(IndexSource src, const void *s, void *d, int64
     LAUNCHCHECK();
 }
 
+// First passes of vectors up to this length claim each tile's slots with one
+// atomic per child, like the later passes, instead of reading the indices
+// once more for the histograms and scanning those.  The children's counters
+// lie kClaimStride words apart, since atomics on one cache line take turns
+// (12 ns each).  us per permute with histograms and with claims: random ints
+// 3 10^6 53 and 44, 17 10^6 178 and 157, 2^25 319 and 319, 2^26 585 and 605,
+// 2^28 2267 and 2401; transposed ones 2^25 324 and 317; random doubles 17 10^6
+// 299 and 274, 2^25 528 and 530, 2^26 994 and 1048.  Claims come in no order,
+// so the ends of neighbouring tiles' runs no longer meet in one XCD's L2.
+constexpr int kClaimStride = 32;
+template <class T>
+constexpr int64_t claim_max() { return sizeof(T) == 4 ? (int64_t)1 << 25 : (int64_t)3 << 23; }
+
 static int64_t up256(int64_t b) { return (b + 255) & ~(int64_t)255; }
 
 // Scratch: two (idx, val) buffers of n pairs and one counter array per
@@ -615,6 +624,8 @@ struct PartLayout {
     uint64_t *status0 = nullptr;
     unsigned *hist0 = nullptr;
     int64_t grid0 = 0;            // tiles of the first pass (one region)
+    bool claim = false;           // the first pass claims its slots
+    int stride0 = 1;              // words between its children's counters
     // Region sizes per pass: from ceil-pow2(n) down to the final block, at
     // most 8 bits per pass; full 8-bit passes first, the odd bits last (the
     // first pass takes its slots from the histogram, later passes claim
@@ -625,7 +636,9 @@ struct PartLayout {
     void clear() const {
         if (clear_to > clear_from) fill_u32((unsigned *)clear_from, 0, (int64_t)(clear_to - clear_from) / 4);
     }
-    PartLayout(int64_t n, void *scratch) {
+    // may_claim: the first pass is k_partition's own (the rank runs the
+    // inverse's itself, from scanned counts)
+    PartLayout(int64_t n, void *scratch, bool may_claim) {
         while (((int64_t)1 << nlog) < n) nlog++;
         if (nlog <= blk_log<T>()) return;   // one block: no scratch
         if (!scratch) usage_error("permute called without scratch");
@@ -648,6 +661,7 @@ struct PartLayout {
         levels = (nlog - blk_log<T>() + 7) / 8;
         // per level: its child counters (>= 256 entries: the column scan
         // writes 256 totals)
+        char *const first = b;
         int pl = nlog;
         for (int l = 0; l < levels; l++) {
             const int cl = pl - bits(l, pl);
@@ -657,13 +671,18 @@ struct PartLayout {
             pl = cl;
         }
         grid0 = (n + kPartTile - 1) / kPartTile;
-        // the column scan's status, or the look-back's tile counter; then the
-        // histogram, or the look-back words (cleared with the counters)
+        // the column scan's status and the histogram, or, when the first pass
+        // claims its slots, its children's counters in the histogram's place
+        claim = may_claim && n <= claim_max<T>();
         status0 = (uint64_t *)b;
         b += up(8 * tile_scan_status_words(grid0));
         hist0 = (unsigned *)b;
-        if (kPartLookback) b += up(4 * (int64_t)kMaxFan * grid0);
-        clear_from = (char *)cnts[0];
+        if (claim) {
+            cnts[0] = hist0;
+            stride0 = kClaimStride;
+            b += 4 * kMaxFan * kClaimStride;
+        }
+        clear_from = first;
         clear_to = b;
     }
 };
@@ -676,6 +695,7 @@ static void partition_later_levels(const PartLayout<T> &L, IndexSource src, void
     int plog = L.nlog;
     for (int l = 0; l < l0; l++) plog -= L.bits(l, plog);
     unsigned *cnt = L.cnts[l0 - 1];
+    int pstride = l0 == 1 ? L.stride0 : 1;
     for (int l = l0; l < L.levels; l++) {
         const int clog = plog - L.bits(l, plog);
         unsigned *const prev = cnt;
@@ -687,13 +707,14 @@ static void partition_later_levels(const PartLayout<T> &L, IndexSource src, void
         const int out = cur == 0 ? 1 : 0;
         if (l + 1 == L.levels)        // children are the final blocks: write Local16
             k_partition<T, false, Local16<T>><<<(unsigned)grid, kPartThreads, 0, g_stream>>>(
-                src, L.buf[cur], nullptr, L.local[out], n, plog, clog, tpr, prev, cnt, nullptr, err);
+                src, L.buf[cur], nullptr, L.local[out], n, plog, clog, tpr, prev, cnt, nullptr, 1, pstride, err);
         else
             k_partition<T, false><<<(unsigned)grid, kPartThreads, 0, g_stream>>>(
-                src, L.buf[cur], nullptr, L.buf[out], n, plog, clog, tpr, prev, cnt, nullptr, err);
+                src, L.buf[cur], nullptr, L.buf[out], n, plog, clog, tpr, prev, cnt, nullptr, 1, pstride, err);
         LAUNCHCHECK();
         cur = out;
         plog = clog;
+        pstride = 1;
     }
     const int64_t blocks = ((n - 1) >> blk_log<T>()) + 1;
     if (L.levels == l0) usage_error("permute: no level after the first");
@@ -715,7 +736,7 @@ static void run_partition(void *d, const void *s, IndexSource src, int64_t n, vo
         else launch_permute_direct<T, 1024, 16>(src, s, d, n, cnt, err);
         return;
     }
-    const PartLayout<T> L(n, scratch);
+    const PartLayout<T> L(n, scratch, true);
     L.clear();
     if (L.levels == 0) {
         k_block_scatter<T, true><<<1, kPartThreads, 0, g_stream>>>(src, Pairs<T>{}, (const T *)s, (T *)d, n, nullptr,
@@ -723,22 +744,17 @@ static void run_partition(void *d, const void *s, IndexSource src, int64_t n, vo
         LAUNCHCHECK();
         return;
     }
-    // first pass: one region, many tiles -> slots from a histogram + column
-    // scan (or the look-back)
+    // first pass: one region, many tiles
     const int plog = L.nlog;
     const int clog = plog - L.bits(0, plog);
-    const int64_t tpr = L.grid0;
-    unsigned *cnt = L.cnts[0];
-    unsigned *hist = (kPartLookback || kPartAtomicFirst) ? nullptr : L.hist0;
-    uint32_t *lb = kPartLookback ? L.hist0 : nullptr;
-    unsigned *lb_ctr = kPartLookback ? (unsigned *)L.status0 : nullptr;
-    if (!kPartLookback && !kPartAtomicFirst) {
+    unsigned *const hist = L.claim ? nullptr : L.hist0;
+    if (!L.claim) {
         k_part_hist<<<(unsigned)L.grid0, kPartThreads, 0, g_stream>>>(src, n, clog, hist);
         LAUNCHCHECK();
-        tile_scan(hist, L.grid0, cnt, L.status0, true);
+        tile_scan(hist, L.grid0, L.cnts[0], L.status0, true);
     }
     k_partition<T, true><<<(unsigned)L.grid0, kPartThreads, 0, g_stream>>>(
-        src, Pairs<T>{}, (const T *)s, L.buf[0], n, plog, clog, tpr, nullptr, cnt, hist, err, lb, lb_ctr);
+        src, Pairs<T>{}, (const T *)s, L.buf[0], n, plog, clog, L.grid0, nullptr, L.cnts[0], hist, L.stride0, 1, err);
     LAUNCHCHECK();
     partition_later_levels<T>(L, src, d, n, 1, 0, err);
 }
@@ -758,7 +774,7 @@ void partition_permute(void *d, const void *s, const int *p, const void *sd, int
 InvertFirstPass partition_invert_begin(int64_t n, void *scratch) {
     InvertFirstPass f{};
     if (n <= 0) return f;
-    const PartLayout<int> L(n, scratch);
+    const PartLayout<int> L(n, scratch, false);
     if (L.levels < 2) return f;          // one partition pass or none: partition_invert
     L.clear();
     f.pairs = L.buf[0].p;
@@ -768,7 +784,7 @@ InvertFirstPass partition_invert_begin(int64_t n, void *scratch) {
 }
 
 void partition_invert_finish(int *rank, int64_t n, void *scratch) {
-    const PartLayout<int> L(n, scratch);   // the layout of partition_invert_begin, counters kept
+    const PartLayout<int> L(n, scratch, false);   // the layout of partition_invert_begin, counters kept
     if (L.levels < 2) usage_error("partition_invert_finish: no split invert for %lld elements", (long long)n);
     // later passes read only the pair buffers; the source is not consulted
     const IndexSource src{nullptr, SegdView(), false, 1, SegdView(), true};

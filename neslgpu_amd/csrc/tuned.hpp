@@ -33,9 +33,6 @@
 #ifndef CVLHIP_BLK_LOG4
 #define CVLHIP_BLK_LOG4 13
 #endif
-#ifndef CVLHIP_PART_ATOMIC_FIRST
-#define CVLHIP_PART_ATOMIC_FIRST 0
-#endif
 #ifndef CVLHIP_RANK_THREADS
 #define CVLHIP_RANK_THREADS 512
 #endif

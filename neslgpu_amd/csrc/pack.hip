@@ -2,11 +2,11 @@
 // (ref nesl/cvl/serial/library.c:51-164; the VCODE PACK driver is
 // nesl/vcode/main.c:577-642).
 //
-// pk2 is one single-pass kernel: each tile loads its flags and values,
-// ranks the true flags with a wave-wide scan of per-lane counts, gets the
-// number of true flags before the tile from the decoupled look-back, and
-// writes the kept values to their final positions.  Input is read once and
-// the output written once.  The segmented pack keeps the flat order
+// pk2: each tile loads its flags and values, ranks the true flags with a
+// wave-wide scan of per-lane counts, gets the number of true flags before the
+// tile -- from a look-back in the same kernel, or, for mid-size vectors, from
+// a count of every tile before it -- and writes the kept values to their final
+// positions.  The segmented pack keeps the flat order
 // (library.c:139-164), so it is the same kernel; pk1_lev, the per-segment
 // counts, is a segmented reduction.
 #include "cvl_hip.hpp"
@@ -42,7 +42,40 @@ struct PackShape {
     static constexpr int TILE = WAVES * WAVE_ELEMS;
 };
 
+// Flags set per tile of k_pack<T, R, B> (COUNTED), whose workgroups then add
+// up the tiles before theirs instead of looking back.
 template <class T, int R, int B>
+__global__ __launch_bounds__(B) void k_pack_count(const int *__restrict__ f, int64_t n, int *__restrict__ counts,
+                                                  int aligned) {
+    using S = PackShape<T, R, B>;
+    typedef int i32x4 __attribute__((ext_vector_type(4)));
+    constexpr int PER = S::TILE / B;
+    static_assert(PER % 4 == 0, "runs of four flags per lane");
+    __shared__ int s_w[S::WAVES];
+    const int64_t t0 = (int64_t)blockIdx.x * S::TILE;
+    int c = 0;
+    if (aligned && t0 + S::TILE <= n) {
+#pragma unroll
+        for (int g = 0; g < PER / 4; g++) {
+            const i32x4 v = *(const i32x4 *)(f + t0 + ((int64_t)g * B + threadIdx.x) * 4);
+            c += (v.x != 0) + (v.y != 0) + (v.z != 0) + (v.w != 0);
+        }
+    } else {
+        for (int64_t k = t0 + threadIdx.x; k < n && k < t0 + S::TILE; k += B) c += f[k] != 0;
+    }
+    c = wave_reduce(c, AddZ());
+    if (threadIdx.x % kWave == 0) s_w[threadIdx.x / kWave] = c;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int tot = 0;
+        for (int i = 0; i < S::WAVES; i++) tot += s_w[i];
+        counts[blockIdx.x] = tot;
+    }
+}
+
+// COUNTED: `status` holds the tiles' counts of k_pack_count (and there is no
+// counter), else look-back status words.
+template <class T, int R, int B, bool COUNTED>
 __global__ __launch_bounds__(B) void k_pack(const T *__restrict__ s, const int *__restrict__ f,
                                                  T *__restrict__ d, int64_t n, int64_t dlim,
                                                  uint64_t *__restrict__ status, unsigned *__restrict__ counter,
@@ -56,13 +89,22 @@ __global__ __launch_bounds__(B) void k_pack(const T *__restrict__ s, const int *
     __shared__ int s_wbase[S::WAVES];
     __shared__ T s_run[S::WAVES][S::ROW];   // one row's kept values, compacted
 
-    if (threadIdx.x == 0) s_tile = counter ? atomicAdd(counter, 1u) : blockIdx.x;   // no counter: one tile
-    __syncthreads();
-    const int64_t tile = s_tile;
+    if constexpr (!COUNTED) {
+        if (threadIdx.x == 0) s_tile = counter ? atomicAdd(counter, 1u) : blockIdx.x;   // no counter: one tile
+        __syncthreads();
+    }
+    const int64_t tile = COUNTED ? (int64_t)blockIdx.x : (int64_t)s_tile;
     const int w = threadIdx.x / kWave;
     const int lane = threadIdx.x % kWave;
     const int64_t wbase = tile * S::TILE + (int64_t)w * S::WAVE_ELEMS + (int64_t)lane * V;
 
+    __shared__ int s_before[S::WAVES];
+    if constexpr (COUNTED) {
+        int before = 0;
+        for (int64_t i = threadIdx.x; i < tile; i += B) before += ((const int *)status)[i];
+        before = wave_reduce(before, add);
+        if (lane == 0) s_before[w] = before;      // read after the barrier below
+    }
     T x[R][V];
     uint32_t fb[R];
     int pos[R];          // rank of the lane's first kept element within the wave
@@ -101,7 +143,10 @@ __global__ __launch_bounds__(B) void k_pack(const T *__restrict__ s, const int *
 #pragma unroll
         for (int i = 0; i < S::WAVES; i++) { wb[i] = tot; tot += s_wcnt[i]; }
         int P = 0;
-        if (tile == 0) {
+        if constexpr (COUNTED) {
+#pragma unroll
+            for (int i = 0; i < S::WAVES; i++) P += s_before[i];
+        } else if (tile == 0) {
             if (lane == 0) TileStatus<int>::publish(status, 0, kPrefix, tot);
         } else {
             if (lane == 0) TileStatus<int>::publish(status, tile, kAggregate, tot);
@@ -159,6 +204,16 @@ int64_t pack_scratch_bytes(int64_t n) {
 template <class T>
 constexpr int pack_block() { return 1024; }
 
+// Vectors of several look-back tiles and at most this length count their
+// flags per tile first and pack in tiles an eighth as large: the flags are
+// read twice, from the caches, but no tile waits for another, nothing is
+// cleared and mid-size vectors reach every CU.  us per PACK (count to the
+// host, then this) against the look-back: ints 40000 20 -> 19, 10^6 23 -> 20, 4
+// 10^6 29 -> 24, 16 10^6 62 -> 56; doubles 10^6 22 -> 20, 8 10^6 50 -> 43, 16
+// 10^6 80 -> 73.  Above, the second reading leaves the caches and each tile
+// adds up more than 4096 counts.
+constexpr int64_t kPackCountedMax = (int64_t)1 << 24;
+
 // Packs the n elements of s whose flag is set into d, which holds dlim.
 template <class T>
 void pack(void *d, const void *s, const void *f, int64_t n, int64_t dlim, void *scratch) {
@@ -168,9 +223,23 @@ void pack(void *d, const void *s, const void *f, int64_t n, int64_t dlim, void *
     if (n <= 0) return;
     if (!scratch) usage_error("pack called without scratch");
     int64_t tiles = (n + S::TILE - 1) / S::TILE;
+    if (tiles > 1 && n <= kPackCountedMax) {
+        constexpr int R = 4;
+        using C = PackShape<T, R, kBlock>;
+        static_assert(8 * C::TILE >= 4 * PackShape<T, kPackRows>::TILE, "the counts fit the status words' scratch");
+        const unsigned g = (unsigned)((n + C::TILE - 1) / C::TILE);
+        int *counts = (int *)((char *)scratch + kPackHeader);
+        k_pack_count<T, R, kBlock><<<g, kBlock, 0, g_stream>>>((const int *)f, n, counts, ((uintptr_t)f & 15) == 0);
+        LAUNCHCHECK();
+        k_pack<T, R, kBlock, true><<<g, kBlock, 0, g_stream>>>(
+            (const T *)s, (const int *)f, (T *)d, n, dlim, (uint64_t *)counts, nullptr,
+            (((uintptr_t)s | (uintptr_t)f) & 15) == 0, device_error_word());
+        LAUNCHCHECK();
+        return;
+    }
     if (tiles > 1) fill_u32(scratch, 0, (kPackHeader + 8 * tiles) / 4);
     int aligned = (((uintptr_t)s | (uintptr_t)f) & 15) == 0;
-    k_pack<T, kPackRows, B><<<(unsigned)tiles, B, 0, g_stream>>>(
+    k_pack<T, kPackRows, B, false><<<(unsigned)tiles, B, 0, g_stream>>>(
         (const T *)s, (const int *)f, (T *)d, n, dlim, (uint64_t *)((char *)scratch + kPackHeader),
         tiles > 1 ? (unsigned *)scratch : nullptr, aligned, device_error_word());
     LAUNCHCHECK();

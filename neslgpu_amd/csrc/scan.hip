@@ -2,7 +2,8 @@
 // (ref nesl/cvl/serial/vprims.c:17-201).
 //
 // Scans are exclusive; segmented scans restart from the identity at every
-// segment.  All of them are single-pass decoupled look-back scans: a tile of
+// segment.  All but mid-size unsegmented scans (launch_scan_aggs) are
+// single-pass decoupled look-back scans: a tile of
 // TILE elements is loaded once with 16-byte lane loads, scanned in registers
 // (lane-sequential, wave-wide DPP scan per row, rows in order, waves
 // combined through LDS), its exclusive prefix comes from the look-back over
@@ -266,12 +267,52 @@ static void launch_scan_r(const void *s, void *d, int64_t n, SegBits sb, void *s
     LAUNCHCHECK();
 }
 
+// Scans of several look-back tiles that stay in the caches fold each tile
+// first (k_tile_aggs) and then scan with every workgroup folding the
+// aggregates before its tile: the values are read twice, but nothing is
+// cleared and no tile waits for another, so tiles can be small enough for
+// every CU to have one.  us per call against the look-back: ints 10^5 9.4 ->
+// 6.1, 10^6 9.8 -> 6.1, 8 10^6 17.2 -> 14.1, but 12 10^6 20.8 -> 23.1; double +
+// 10^6 14.5 -> 6.8, 8 10^6 46 -> 31, 20 10^6 105 -> 75, double max 82 -> 76, but
+// 25 10^6 101 -> 113 (+ 125 -> 111): the second reading then leaves the caches.
+// Double sums come closer to exact ones: the aggregates fold in a tree, not
+// one by one (2^25 values off by 1.1e-15 before, 2.8e-16 so, of the 2-norm).
+template <class Op>
+constexpr int64_t scan_aggs_max() { return sizeof(typename Op::T) == 4 ? (int64_t)1 << 23 : (int64_t)20 << 20; }
+
+template <class Op>
+static void launch_scan_aggs(const void *s, void *d, int64_t n, void *scratch) {
+    using T = typename Op::T;
+    constexpr int R = 4, B = 512;
+    using S = ScanShape<Op, R, B>;
+    static_assert((int64_t)S::TILE * TileStatus<T>::kWords * 8 >= (int64_t)sizeof(T) * ScanShape<Op, kScanRows>::TILE,
+                  "the aggregates fit the status words' scratch");
+    if (!scratch) { usage_error("scan of %lld elements called without scratch", (long long)n); return; }
+    const unsigned tiles = (unsigned)((n + S::TILE - 1) / S::TILE);
+    T *aggs = (T *)((char *)scratch + kScanHeaderBytes);
+    k_tile_aggs<Op, R, B><<<tiles, B, 0, g_stream>>>((const T *)s, n, al16(s), aggs);
+    LAUNCHCHECK();
+    k_scan<Op, R, false, false, ArrayIn<T>, B, false, 16, true><<<tiles, B, 0, g_stream>>>(
+        ArrayIn<T>{(const T *)s}, (T *)d, n, SegBits{nullptr, nullptr, nullptr}, (uint64_t *)aggs, nullptr,
+        al16(s) && al16(d), device_error_word());
+    LAUNCHCHECK();
+}
+
 // The CVL entry points: scratch_bytes counts tiles of kBlock threads and
 // kScanRows rows, so the tiles launched must not be smaller.
 template <class Op, bool SEG, bool REDUCE>
 static void launch_scan(const void *s, void *d, int64_t n, SegBits sb, void *scratch, unsigned *err = nullptr) {
-    constexpr int R = scan_rows<Op, SEG, REDUCE>();
-    static_assert(scan_block<Op, SEG, REDUCE>() * R >= kBlock * kScanRows, "scratch sizes count the most tiles");
+    constexpr int R = scan_rows<Op, SEG, REDUCE>(), B = scan_block<Op, SEG, REDUCE>();
+    static_assert(B * R >= kBlock * kScanRows, "scratch sizes count the most tiles");
+    if constexpr (!REDUCE) {
+        // one tile holds it: no more rows than it needs (1000 ints 6.4 -> 4.1
+        // us, 1000 doubles 6.0 -> 3.4-4.4)
+        if (n <= ScanShape<Op, 1, 1024>::TILE) return launch_scan_r<Op, 1, SEG, false, 1024>(s, d, n, sb, scratch, err);
+        if (n <= ScanShape<Op, 4, 1024>::TILE) return launch_scan_r<Op, 4, SEG, false, 1024>(s, d, n, sb, scratch, err);
+    }
+    if constexpr (!SEG && !REDUCE) {
+        if (n > ScanShape<Op, R, B>::TILE && n <= scan_aggs_max<Op>()) return launch_scan_aggs<Op>(s, d, n, scratch);
+    }
     launch_scan_r<Op, R, SEG, REDUCE>(s, d, n, sb, scratch, err);
 }
 

@@ -161,11 +161,14 @@ struct NolbRecords {
 // NolbRecords of gridDim.x tiles and k_seg_reduce_fix finishes the
 // segments that cross tiles.
 //
+// AGGS (unsegmented scans only): no look-back; `status` holds the aggregates
+// of all tiles (k_tile_aggs), and the workgroup folds those before its own.
+//
 // scan_tile is the work of one workgroup on one tile (`tile` of `ntiles`;
 // NOLB records are laid out for ntiles tiles).  k_scan runs one tile per
 // workgroup; the segmented-op schedules (k_seg_sched) loop over tiles.
 
-template <class Op, int R, bool SEG, bool REDUCE, class In, int B, bool NOLB, int VB = 16>
+template <class Op, int R, bool SEG, bool REDUCE, class In, int B, bool NOLB, int VB = 16, bool AGGS = false>
 __device__ __forceinline__ void scan_tile(const In &in, typename Op::T *__restrict__ out, int64_t n, SegBits sb,
                                           uint64_t *__restrict__ status, int64_t tile, int64_t ntiles,
                                           bool aligned, unsigned *__restrict__ err) {
@@ -176,6 +179,7 @@ __device__ __forceinline__ void scan_tile(const In &in, typename Op::T *__restri
     constexpr uint32_t VMASK = (1u << V) - 1u;
     static_assert(!NOLB || (SEG && REDUCE), "only segmented reductions run without look-back");
     static_assert(VB == 16 || (SEG && REDUCE), "wide lanes only in segmented reductions");
+    static_assert(!AGGS || !SEG, "tile aggregates carry no head flags");
     const Op op;
 
     __shared__ T s_wagg[S::WAVES];
@@ -219,6 +223,16 @@ __device__ __forceinline__ void scan_tile(const In &in, typename Op::T *__restri
     }
 #pragma unroll
     for (int r = 0; r < R; r++) in.template load<Op, V>(wbase + (int64_t)r * S::ROW, n, aligned, x[r]);
+    __shared__ T s_before[AGGS ? S::WAVES : 1];
+    if constexpr (AGGS) {
+        // in tile order: consecutive tiles per thread, then lanes, then waves
+        const int64_t per = (tile + B - 1) / B;
+        T before = Op::neutral();
+        for (int64_t i = threadIdx.x * per; i < tile && i < (threadIdx.x + 1) * per; i++)
+            before = op(before, ((const T *)status)[i]);
+        before = wave_reduce(before, op);
+        if (lane == 0) s_before[w] = before;     // read after the barrier below
+    }
     // The tile's head bitmap words (and, for reductions, head counts) are
     // staged in LDS with one coalesced pass, so the rows below read them
     // there instead of with two more vector loads each.  Words past the
@@ -338,7 +352,10 @@ __device__ __forceinline__ void scan_tile(const In &in, typename Op::T *__restri
             tf |= f;
         }
         T P = Op::neutral();
-        if constexpr (NOLB) {
+        if constexpr (AGGS) {
+#pragma unroll
+            for (int i = 0; i < S::WAVES; i++) P = op(P, s_before[i]);
+        } else if constexpr (NOLB) {
             if (lane == 0) {
                 const NolbRecords<T> rec = NolbRecords<T>::at(status, ntiles);
                 rec.agg[tile] = tv;
@@ -413,7 +430,7 @@ __device__ __forceinline__ void scan_tile(const In &in, typename Op::T *__restri
 }
 
 template <class Op, int R, bool SEG, bool REDUCE, class In = ArrayIn<typename Op::T>, int B = kBlock,
-          bool NOLB = false, int VB = 16>
+          bool NOLB = false, int VB = 16, bool AGGS = false>
 __global__ __launch_bounds__(B) void k_scan(In in, typename Op::T *__restrict__ out, int64_t n, SegBits sb,
                                             uint64_t *__restrict__ status, unsigned *__restrict__ counter,
                                             int aligned_i, unsigned *__restrict__ err) {
@@ -422,8 +439,41 @@ __global__ __launch_bounds__(B) void k_scan(In in, typename Op::T *__restrict__ 
     // single-tile launch passes no counter
     if (threadIdx.x == 0) s_tile = counter ? atomicAdd(counter, 1u) : blockIdx.x;
     __syncthreads();
-    scan_tile<Op, R, SEG, REDUCE, In, B, NOLB, VB>(in, out, n, sb, status, (int64_t)s_tile, (int64_t)gridDim.x,
-                                                   aligned_i != 0, err);
+    scan_tile<Op, R, SEG, REDUCE, In, B, NOLB, VB, AGGS>(in, out, n, sb, status, (int64_t)s_tile, (int64_t)gridDim.x,
+                                                         aligned_i != 0, err);
+}
+
+// aggs[t]: the fold of tile t of a k_scan with AGGS (R rows, B threads).
+template <class Op, int R, int B>
+__global__ __launch_bounds__(B) void k_tile_aggs(const typename Op::T *__restrict__ in, int64_t n, int aligned_i,
+                                                 typename Op::T *__restrict__ aggs) {
+    using T = typename Op::T;
+    using S = ScanShape<Op, R, B>;
+    constexpr int V = S::V;
+    const Op op;
+    __shared__ T s_w[S::WAVES];
+    const int w = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+    const int64_t wbase = (int64_t)blockIdx.x * S::TILE + (int64_t)w * S::WAVE_ELEMS + (int64_t)lane * V;
+    T x[R][V];
+#pragma unroll
+    for (int r = 0; r < R; r++) load_lane<Op, V>(in, wbase + (int64_t)r * S::ROW, n, aligned_i != 0, x[r]);
+    T acc = Op::neutral();
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        T a = x[r][0];
+#pragma unroll
+        for (int k = 1; k < V; k++) a = op(a, x[r][k]);
+        if constexpr (ordered<Op>::value) acc = op(acc, wave_reduce(a, op));
+        else acc = op(acc, a);
+    }
+    if constexpr (!ordered<Op>::value) acc = wave_reduce(acc, op);
+    if (lane == 0) s_w[w] = acc;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        T b = s_w[0];
+        for (int i = 1; i < S::WAVES; i++) b = op(b, s_w[i]);
+        aggs[blockIdx.x] = b;
+    }
 }
 
 // Rows per wave, threads per workgroup and bytes per lane and row of the

@@ -108,7 +108,15 @@ struct SegBits {
     const int *nz;
     const void *sd;          // when set (and heads null): read the rest from this descriptor's header
     int64_t m;               // segment count, when known (0: unknown); lets reductions see that nz is the identity
+    const int *empties;      // lengths, when the reduction's kernel also writes the identities of empty segments
 };
+
+// The identity for every empty segment of a reduction, by the whole grid.
+template <class Op>
+__device__ __forceinline__ void write_empties(typename Op::T *__restrict__ out, const int *__restrict__ lens, int64_t m) {
+    for (int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; g < m; g += (int64_t)gridDim.x * blockDim.x)
+        if (lens[g] == 0) out[g] = Op::cvl_id();
+}
 
 // Where a scan's input comes from: an array (ArrayIn), or -- in generated
 // fused operations -- an expression evaluated per element.
@@ -441,6 +449,8 @@ __global__ __launch_bounds__(B) void k_scan(In in, typename Op::T *__restrict__ 
     __syncthreads();
     scan_tile<Op, R, SEG, REDUCE, In, B, NOLB, VB, AGGS>(in, out, n, sb, status, (int64_t)s_tile, (int64_t)gridDim.x,
                                                          aligned_i != 0, err);
+    if constexpr (NOLB)
+        if (sb.empties) write_empties<Op>(out, sb.empties, sb.m);
 }
 
 // aggs[t]: the fold of tile t of a k_scan with AGGS (R rows, B threads).

@@ -238,15 +238,18 @@ __device__ __forceinline__ int sched_arm_of(const void *sd) {
 
 // sv: the descriptor's view as the host knows it, or (from_hdr) read here
 // from the descriptor `sd` itself.  arm < 0: the descriptor's pick.
+// empties (reductions): also write the identities of empty segments.
 template <class Op, bool REDUCE, class In>
 __global__ __launch_bounds__((sched_block<Op, REDUCE>())) void k_seg_sched(In in, typename Op::T *__restrict__ out,
                                                                           int64_t n, SegdView sv, const void *sd,
                                                                           int from_hdr, void *scratch, int aligned_i,
-                                                                          unsigned *err, int arm) {
+                                                                          unsigned *err, int arm, int empties) {
     constexpr int B = sched_block<Op, REDUCE>();
+    if constexpr (REDUCE)
+        if (empties) write_empties<Op>(out, sv.lens, sv.m);
     if (from_hdr) sv = SegdView::from_header(sd);
     if (arm < 0) arm = sched_arm_of<Op, REDUCE>(sd);
-    const SegBits sb{sv.heads, sv.wcnt, sv.nz, nullptr, sv.m};
+    const SegBits sb{sv.heads, sv.wcnt, sv.nz, nullptr, sv.m, nullptr};
     const bool aligned = aligned_i != 0;
     switch (arm) {
     case kArmFlat2: sched_flat<Op, 2, REDUCE, In, B, true>(in, out, n, sb, scratch, aligned, err); return;
@@ -297,21 +300,24 @@ inline int sched_grid(int64_t n) {
 }
 
 // The segmented reduction of the CVL entries and of generated fused
-// operations, after the identities of empty segments are written.  Vectors
+// operations, after the identities of empty segments are written, or, with
+// `empties` (sv given, no more segments than elements, so that each thread
+// looks at few), together with them: a launch less.  Vectors
 // shorter than kSchedMinN (their descriptors carry no pick) run the fixed
 // schedule one tile per workgroup; longer ones, or a forced arm, run
 // k_seg_sched and its second step.  Scratch: sched_scratch_bytes<Op, true>.
 template <class Op, class In>
 inline void seg_reduce_run(const In &in, typename Op::T *out, int64_t n, const SegdView &sv, const void *sd,
-                           bool from_hdr, void *scratch, bool aligned, unsigned *err, int arm, hipStream_t st) {
+                           bool from_hdr, void *scratch, bool aligned, unsigned *err, int arm, hipStream_t st,
+                           bool empties = false) {
     using T = typename Op::T;
     if (n <= 0) return;
     if (arm < 0 && n < kSchedMinN) {
         using S = ScanShape<Op, kSegReduceRows, kSegReduceBlock, kSegReduceLaneBytes>;
         const int64_t tiles = (n + S::TILE - 1) / S::TILE;
         void *recs = (char *)scratch + kSchedHeader;
-        const SegBits sb = from_hdr ? SegBits{nullptr, nullptr, nullptr, sd, 0}
-                                    : SegBits{sv.heads, sv.wcnt, sv.nz, nullptr, sv.m};
+        const SegBits sb = from_hdr ? SegBits{nullptr, nullptr, nullptr, sd, 0, nullptr}
+                                    : SegBits{sv.heads, sv.wcnt, sv.nz, nullptr, sv.m, empties ? sv.lens : nullptr};
         k_scan<Op, kSegReduceRows, true, true, In, kSegReduceBlock, true, kSegReduceLaneBytes>
             <<<(unsigned)tiles, kSegReduceBlock, 0, st>>>(
             in, out, n, sb, (uint64_t *)recs, nullptr, aligned, err);
@@ -319,7 +325,7 @@ inline void seg_reduce_run(const In &in, typename Op::T *out, int64_t n, const S
         return;
     }
     k_seg_sched<Op, true, In><<<sched_grid<Op, true, In>(n), sched_block<Op, true>(), 0, st>>>(
-        in, out, n, sv, sd, from_hdr ? 1 : 0, scratch, aligned ? 1 : 0, err, arm);
+        in, out, n, sv, sd, from_hdr ? 1 : 0, scratch, aligned ? 1 : 0, err, arm, empties ? 1 : 0);
     k_seg_reduce_fix_sched<Op><<<1, kFixThreads, 0, st>>>(scratch, out);
 }
 

@@ -38,7 +38,11 @@ __device__ __forceinline__ float sched_feature(int i, int64_t n, int64_t m, cons
 }
 
 // Schedules a descriptor admits whatever the network predicts.  The flat
-// schedules (0-2) take any descriptor.  The per-segment ones (3 thread, 4
+// 8-row schedule (0) takes any descriptor.  The others exist for vectors
+// whose 8-row tiles leave CUs idle, and are admitted below 2^kOthersMaxLogN
+// elements only, the largest length the network was trained on (8 rows are
+// the fastest there; at 2^28 ints in geometric(256) segments a network's pick
+// of 2 rows took 0.84 ms against 0.47).  The per-segment ones (3 thread, 4
 // wave, 5 workgroup) give a segment one lane, wave or workgroup: one long
 // segment serialises them and a few segments leave the chip idle, so each
 // is admitted only when the longest segment is below 2^(kArmMaxClass + 1)
@@ -46,7 +50,9 @@ __device__ __forceinline__ float sched_feature(int i, int64_t n, int64_t m, cons
 // length class holding a segment (-1: none).  Bit a set: schedule a admitted.
 constexpr int kArmMaxClass[3] = {5, 12, 15};
 constexpr int kArmMinLogM[3] = {14, 11, 9};
-__host__ __device__ inline unsigned sched_admitted(int cmax, int64_t m) {
+constexpr int kOthersMaxLogN = 25;
+__host__ __device__ inline unsigned sched_admitted(int cmax, int64_t n, int64_t m) {
+    if (n >= ((int64_t)1 << kOthersMaxLogN)) return 1u;
     unsigned a = 7u;
     for (int k = 0; k < 3; k++)
         if (cmax <= kArmMaxClass[k] && m >= ((int64_t)1 << kArmMinLogM[k])) a |= 1u << (3 + k);

@@ -135,3 +135,16 @@ def test_descriptor_edges(cv, name, lens):
     assert np.array_equal(hist[:21], np.bincount(cls, lens64[nz], 21)[:21])
     assert np.array_equal(hist[21:], np.bincount(cls, minlength=21))
     assert cv.lib.cvlhip_check_device_errors() == 0
+
+
+@pytest.mark.parametrize("n", [(1 << 25) - 1, 1 << 25, 1 << 28])
+def test_long_vectors_keep_the_widest_tiles(cv, n):
+    """From 2^25 elements on a descriptor's picks are the 8-row schedule."""
+    m = n // 256
+    lens = np.full(m, 256, np.int32)
+    lens[-1] += n - m * 256
+    sd = cv.segd(lens)
+    picks = [cv.lib.cvlhip_segd_pick(sd, red, size) for red in (0, 1) for size in (4, 8)]
+    print("picks", n, picks, flush=True)
+    if n >= 1 << 25 and cv.lib.cvlhip_sched_has_model():
+        assert picks == [0, 0, 0, 0]

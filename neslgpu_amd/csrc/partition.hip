@@ -214,8 +214,8 @@ __device__ __forceinline__ unsigned bucket_place(unsigned *hist, int d, bool run
 // Each tile's slot in each child comes from tile_ofs (the column scan of
 // per-tile histograms: long first passes) or is claimed with one atomic per
 // non-empty child.  cstride, pstride: words from one child's counter to the
-// next, in cnt and prev_cnt.
-template <class T, bool FIRST, class Out = Pairs<T>>
+// next, in cnt and prev_cnt.  RUNS: look for waves of one bucket.
+template <class T, bool FIRST, class Out = Pairs<T>, bool RUNS = sizeof(T) == 4>
 __global__ __launch_bounds__(kPartThreads) void k_partition(IndexSource src, Pairs<T> in,
                                                             const T *__restrict__ in_val, Out out,
                                                             int64_t n, int plog, int clog,
@@ -307,7 +307,7 @@ __global__ __launch_bounds__(kPartThreads) void k_partition(IndexSource src, Pai
 #pragma unroll
     for (int j = 0; j < kPartItems; j++) {
         dg[j] = -1;
-        if (PACKED && j % kPartV == 0) runs = wave_same((int)(qv[j] >> clog));
+        if (RUNS && j % kPartV == 0) runs = wave_same((int)(qv[j] >> clog));
         if (has[j]) {
             const int64_t qq = qv[j];
             const int64_t child = qq >> clog;
@@ -689,7 +689,7 @@ struct PartLayout {
 
 // Levels l0 .. levels-1 after the first (their input: buffer `cur`, its
 // children counted in cnts[l0 - 1]), then the block scatter into d.
-template <class T>
+template <class T, bool RUNS = sizeof(T) == 4>
 static void partition_later_levels(const PartLayout<T> &L, IndexSource src, void *d, int64_t n, int l0, int cur,
                                    unsigned *err) {
     int plog = L.nlog;
@@ -706,10 +706,10 @@ static void partition_later_levels(const PartLayout<T> &L, IndexSource src, void
         const int64_t grid = regions * tpr;
         const int out = cur == 0 ? 1 : 0;
         if (l + 1 == L.levels)        // children are the final blocks: write Local16
-            k_partition<T, false, Local16<T>><<<(unsigned)grid, kPartThreads, 0, g_stream>>>(
+            k_partition<T, false, Local16<T>, RUNS><<<(unsigned)grid, kPartThreads, 0, g_stream>>>(
                 src, L.buf[cur], nullptr, L.local[out], n, plog, clog, tpr, prev, cnt, nullptr, 1, pstride, err);
         else
-            k_partition<T, false><<<(unsigned)grid, kPartThreads, 0, g_stream>>>(
+            k_partition<T, false, Pairs<T>, RUNS><<<(unsigned)grid, kPartThreads, 0, g_stream>>>(
                 src, L.buf[cur], nullptr, L.buf[out], n, plog, clog, tpr, prev, cnt, nullptr, 1, pstride, err);
         LAUNCHCHECK();
         cur = out;
@@ -788,7 +788,8 @@ void partition_invert_finish(int *rank, int64_t n, void *scratch) {
     if (L.levels < 2) usage_error("partition_invert_finish: no split invert for %lld elements", (long long)n);
     // later passes read only the pair buffers; the source is not consulted
     const IndexSource src{nullptr, SegdView(), false, 1, SegdView(), true};
-    partition_later_levels<int>(L, src, rank, n, 1, 0, device_error_word());
+    // (a sort order has no runs to look for: 12 10^6 keys 335 -> 332 us)
+    partition_later_levels<int, false>(L, src, rank, n, 1, 0, device_error_word());
 }
 
 void partition_invert(int *rank, const int *order, int64_t n, const void *sd, int64_t m, void *scratch) {

@@ -922,30 +922,65 @@ __global__ void k_rank_identity(int *rank, int64_t n, SegdView seg, int segmente
 }
 
 // ---------------------------------------------------------------- host driver
+// Up to this many keys the tiles' counts are grouped (no column scans), pass
+// 0 runs without waiting for the host, and the last pass stores the ranks
+// directly: one scattered 4-byte store per key, which stays in the caches
+// while the result is small, in place of the inverse's four or five launches.
+// us per call against the column scans and the partitioned inverse: 17000
+// ints 96 -> 44, 250000 101 -> 51, 10^6 116 -> 72, 3 10^6 152 -> 114, 5 10^6
+// 191 -> 171, 8 10^6 246 -> 236; 250000 doubles 182 -> 105, 3 10^6 303 -> 247,
+// 8 10^6 620 -> 592.  Above, a pass would add up more than kRankGroups
+// groups per tile, and the scattered stores miss the caches.
+constexpr int64_t kRankDirectMax = (int64_t)kRankGroups * kRankGroup * kRankTile;
+// Up to this many keys tiles are small: 250000 ints 51 against 57 us, 500000
+// 57 against 62, but 10^6 75 against 72.
+constexpr int64_t kRankSmallMax = (int64_t)1 << 19;
+constexpr int kRankSmallTile = kRankSmallThreads * kRankSmallItems;
+static_assert(kRankSmallMax <= (int64_t)kRankGroups * kRankGroup * kRankSmallTile, "small tiles are grouped");
+constexpr int kRankPasses = 12;           // most passes: 8 of a double, 4 of a segment number
+
+// Byte offsets of the areas in a rank's scratch.  Every area's whole size is
+// counted, rows of 256 words per tile, group and pass rounded up as the
+// kernels write them; areas that share their bytes are never in use together.
 struct RankScratch {
     int64_t keysA, keysB, idxA, idxB, hist, starts, counters, status, scan_status, status2, orparts, invert, bytes;
+    int64_t groups;                                    // grouped tiles of kRankTile: the group counts of each pass
+    int64_t small_counts, small_groups, small_orparts;   // small tiles: tile counts, group counts, OR words
     RankScratch(int64_t n, bool dbl) {
         auto up = [](int64_t b) { return (b + 255) & ~(int64_t)255; };
-        int64_t kw = dbl ? 8 : 4;
-        int64_t tiles = (n + kRankTile - 1) / kRankTile;
+        auto most = [](int64_t a, int64_t b) { return a > b ? a : b; };
+        auto parts = [](int64_t k, int64_t size) { return (k + size - 1) / size; };
+        constexpr int64_t row = 4 * kRadix;
+        const int64_t kw = dbl ? 8 : 4;
+        const int64_t tiles = most(parts(n, kRankTile), 1);
         keysA = 0;
         keysB = up(keysA + kw * n);
         idxA = up(keysB + kw * n);
         idxB = up(idxA + 4 * n);
         hist = up(idxB + 4 * n);
-        starts = up(hist + 4 * 12 * kRadix);
-        counters = up(starts + 4 * 12 * kRadix);
+        starts = up(hist + kRankPasses * row);
+        counters = up(starts + kRankPasses * row);
         status = up(counters + 4 * 16);
-        scan_status = up(status + 4 * kRadix * (tiles > 0 ? tiles : 1));
-        // one column-scan status region per pass (at most 12), one for the
-        // fused last pass's child counts and one for the speculative first
-        // pass, cleared together
-        status2 = up(scan_status + 14 * 8 * tile_scan_status_words(tiles > 0 ? tiles : 1));
+        // one column-scan status region per pass, one for the fused last
+        // pass's child counts and one for the speculative first pass, cleared
+        // together; grouped tiles have no column scan and keep their group
+        // counts there
+        groups = scan_status = up(status + row * tiles);
+        int64_t scan_bytes = (kRankPasses + 2) * 8 * tile_scan_status_words(tiles);
+        if (n <= kRankDirectMax) scan_bytes = most(scan_bytes, kRankPasses * row * parts(tiles, kRankGroup));
         // the fused last pass's per-tile child counts; the first pass's
         // per-tile OR words
-        orparts = up(status2 + 4 * kRadix * (tiles > 0 ? tiles : 1));
-        invert = up(orparts + 8 * (tiles > 0 ? tiles : 1));
+        status2 = up(scan_status + scan_bytes);
+        orparts = up(status2 + row * tiles);
+        // the inverse's scratch.  Small tiles' counts lie in it: their passes
+        // are done before an inverse (or none) runs.
+        invert = up(orparts + 8 * tiles);
         bytes = up(invert + partition_permute_scratch_bytes(n, 4));
+        const int64_t small_tiles = most(parts(n, kRankSmallTile), 1);
+        small_counts = invert;
+        small_groups = small_counts + row * small_tiles;
+        small_orparts = small_groups + kRankPasses * row * parts(small_tiles, kRankGroup);
+        if (n <= kRankSmallMax) bytes = most(bytes, up(small_orparts + 8 * small_tiles));
     }
 };
 
@@ -986,20 +1021,6 @@ static void launch_grouped(const PassArgs &a, int64_t tiles, bool dbl, bool last
     LAUNCHCHECK();
 }
 
-// Up to this many keys the tiles' counts are grouped (no column scans), pass
-// 0 runs without waiting for the host, and the last pass stores the ranks
-// directly: one scattered 4-byte store per key, which stays in the caches
-// while the result is small, in place of the inverse's four or five launches.
-// us per call against the column scans and the partitioned inverse: 17000
-// ints 96 -> 44, 250000 101 -> 51, 10^6 116 -> 72, 3 10^6 152 -> 114, 5 10^6
-// 191 -> 171, 8 10^6 246 -> 236; 250000 doubles 182 -> 105, 3 10^6 303 -> 247,
-// 8 10^6 620 -> 592.  Above, a pass would add up more than kRankGroups
-// groups per tile, and the scattered stores miss the caches.
-constexpr int64_t kRankDirectMax = (int64_t)kRankGroups * kRankGroup * kRankTile;
-// Up to this many keys tiles are small: 250000 ints 51 against 57 us, 500000
-// 57 against 62, but 10^6 75 against 72.
-constexpr int64_t kRankSmallMax = (int64_t)1 << 19;
-
 void rank_run(int *rank, const void *s, int64_t n, bool dbl, bool up, const void *sd, int64_t m, void *scratch) {
     if (n <= 0) return;
     if (!scratch) usage_error("rank called without scratch");
@@ -1025,26 +1046,16 @@ void rank_run(int *rank, const void *s, int64_t n, bool dbl, bool up, const void
 
     const bool chain = kRankChain && n < (int64_t)kChainMask;
     const bool aligned = ((uintptr_t)s & 15) == 0;
-    // Short vectors are ranked in small tiles, whose counts lie in the
-    // inverse's scratch (n bytes and n / 32 per pass of its 16 n): a direct
-    // inverse needs none.
     const bool grouped = !chain && n <= kRankDirectMax;
     const bool small = grouped && n <= kRankSmallMax;
-    static_assert(kRankSmallMax <= (int64_t)kRankGroups * kRankGroup * kRankSmallThreads * kRankSmallItems,
-                  "small tiles are grouped");
-    const int tile = small ? kRankSmallThreads * kRankSmallItems : kRankTile;
+    const int tile = small ? kRankSmallTile : kRankTile;
     const int64_t tiles = (n + tile - 1) / tile;
     const int64_t ngroups = (tiles + kRankGroup - 1) / kRankGroup;
     const int64_t sw = tile_scan_status_words((n + kRankTile - 1) / kRankTile);
-    unsigned *tile_ofs = (unsigned *)(b + L.status);
+    unsigned *tile_ofs = (unsigned *)(b + (small ? L.small_counts : L.status));
     uint64_t *scan_status = (uint64_t *)(b + L.scan_status);
-    uint32_t *or_parts = (uint32_t *)(b + L.orparts);
-    unsigned *groups = (unsigned *)scan_status;             // ngroups x 256 per pass, in the space of its scan status
-    if (small) {
-        tile_ofs = (unsigned *)(b + L.invert);
-        groups = tile_ofs + kRadix * tiles;
-        or_parts = groups + 12 * kRadix * ngroups;
-    }
+    uint32_t *or_parts = (uint32_t *)(b + (small ? L.small_orparts : L.orparts));
+    unsigned *groups = (unsigned *)(b + (small ? L.small_groups : L.groups));      // ngroups x 256 per pass
     int gs = grid_for(m, kBlock);
     if (gs > 4096) gs = 4096;
     bool runs[12] = {};

@@ -46,3 +46,21 @@ def fp_add_tol_vec(absprefix, seglen):
 def seg_lengths_per_element(lens):
     lens = np.asarray(lens, np.int64)
     return np.repeat(lens, lens)
+
+
+class Guarded:
+    """Scratch of exactly the promised units, followed by a guard that no
+    kernel may write: use it as the call's scratch, then call check()."""
+    GUARD = 32 << 10
+
+    def __init__(self, cv, units):
+        import torch
+        self.nbytes = 8 * int(units)
+        self.buf = torch.full((self.nbytes + self.GUARD,), 0xA5, dtype=torch.uint8, device=cv.device)
+
+    def data_ptr(self):
+        return self.buf.data_ptr()
+
+    def check(self, what=""):
+        bad = (self.buf[self.nbytes:] != 0xA5).nonzero()
+        assert bad.numel() == 0, f"{what}: {bad.numel()} bytes written past the scratch, first at +{int(bad[0])}"

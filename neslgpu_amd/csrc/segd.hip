@@ -304,12 +304,13 @@ __global__ __launch_bounds__(kSmallThreads) void k_segd_scan_sums(uint64_t *part
 }
 
 // `scanned`: parts holds exclusive sums, else the tiles' own.  Of wcnt it
-// writes the first word of each chunk and the last, the number of all heads.
+// writes the first word of each chunk; *count: the number of non-empty
+// segments.
 __global__ __launch_bounds__(kTileThreads) void k_segd_offsets(const int *__restrict__ lens_in, SegdHeader *hdr,
                                                                 int *lens, int *offs, int *nz,
                                                                 int *__restrict__ wcnt,
                                                                 const uint64_t *__restrict__ parts, int scanned,
-                                                                int64_t n, int64_t m) {
+                                                                int *__restrict__ count, int64_t n, int64_t m) {
     constexpr int W = kTileThreads / kWave;
     __shared__ uint64_t s_wave[W];
     __shared__ unsigned s_hist[kHist * kHistCopies];
@@ -339,9 +340,12 @@ __global__ __launch_bounds__(kTileThreads) void k_segd_offsets(const int *__rest
     __syncthreads();
     if (lane == kWave - 1) s_wave[w] = inc;
     __syncthreads();
+    uint64_t through = P;                       // this tile and those before it
 #pragma unroll
-    for (int i = 0; i < W; i++)
+    for (int i = 0; i < W; i++) {
+        through = op(through, s_wave[i]);
         if (i < w) P = op(P, s_wave[i]);
+    }
     uint64_t ex = shfl_up1(inc);
     if (lane == 0) ex = 0;
     P = op(P, ex);
@@ -394,14 +398,21 @@ __global__ __launch_bounds__(kTileThreads) void k_segd_offsets(const int *__rest
         if (only) hdr->hist[tid] = h;
         else if (h) atomicAdd(&hdr->hist[tid], h);
     }
-    if (tile == (int64_t)gridDim.x - 1 && tid == kTileThreads - 1) {
-        const uint64_t all = op(P, sum);
-        offs[m] = (int)(uint32_t)all;
-        wcnt[(n + 31) >> 5] = (int)(all >> 32);
-        hdr->n = n;
-        hdr->m = m;
-        hdr->stats = kStatsMagic;
-        if (only) hdr->sched = 0u;
+    if (tile == (int64_t)gridDim.x - 1) {
+        // chunks that start past the last segment's end (lengths that sum to
+        // less than n): all heads are before them
+        const int end = (int)(uint32_t)through;
+        if (end >= 0)
+            for (int64_t j = end / kChunk + 1 + tid; j * kChunk < n; j += kTileThreads)
+                wcnt[j * kChunkWords] = (int)(through >> 32);
+        if (tid == 0) {
+            offs[m] = end;
+            *count = (int)(through >> 32);
+            hdr->n = n;
+            hdr->m = m;
+            hdr->stats = kStatsMagic;
+            if (only) hdr->sched = 0u;
+        }
     }
     if (tile == 0 && tid == 0 && n > 0) wcnt[0] = 0;
 }
@@ -412,8 +423,9 @@ __global__ __launch_bounds__(kTileThreads) void k_segd_offsets(const int *__rest
 // launch has one workgroup more than chunks, and that last workgroup picks
 // the schedules from the histogram k_segd_offsets completed.
 __global__ __launch_bounds__(kChunkThreads) void k_segd_words(const int *__restrict__ offs, const int *__restrict__ nz,
-                                                             int *wcnt, uint32_t *heads, int64_t words, int64_t chunks,
-                                                             SegdHeader *hdr, int64_t n, int64_t m, int pick) {
+                                                             const int *__restrict__ count, int *wcnt, uint32_t *heads,
+                                                             int64_t words, int64_t chunks, SegdHeader *hdr, int64_t n,
+                                                             int64_t m, int pick) {
     constexpr int W = kChunkWords / kWave;
     __shared__ __attribute__((aligned(16))) unsigned char s_mark[kChunk];
     __shared__ unsigned s_wave[W];
@@ -425,9 +437,9 @@ __global__ __launch_bounds__(kChunkThreads) void k_segd_words(const int *__restr
         return;
     }
     const int64_t w0 = c * kChunkWords, next = w0 + kChunkWords;
-    const int all = wcnt[words];
+    const int all = *count;
     int r0 = n > 0 ? wcnt[w0] : 0, r1 = next < words ? wcnt[next] : all;
-    // (lengths that do not sum to n leave some of these unwritten: clamp)
+    // (negative lengths, or sums that wrap, leave some of these unwritten: clamp)
     r0 = r0 < 0 ? 0 : (r0 > all ? all : r0);
     r1 = r1 > all ? all : r1;
     for (int i = tid; i < kChunk / 16; i += kChunkThreads) ((u32x4 *)s_mark)[i] = u32x4{0u, 0u, 0u, 0u};
@@ -461,12 +473,16 @@ __global__ __launch_bounds__(kChunkThreads) void k_segd_words(const int *__restr
         if (i < w) base += s_wave[i];
     if (w0 + tid < words) {
         heads[w0 + tid] = h;
-        if (tid > 0) wcnt[w0 + tid] = (int)base;
+        wcnt[w0 + tid] = (int)base;          // the first word's: the clamped count
     }
-    if (c == chunks - 1 && tid < 8) heads[words + tid] = 0u;
+    if (c == chunks - 1) {
+        if (tid < 8) heads[words + tid] = 0u;
+        if (tid == kChunkWords - 1) wcnt[words] = (int)(base + cnt);     // all heads
+    }
 }
 
-// 16 bytes per kSmallSegd lengths hold the tile sums.
+// The count of non-empty segments, then, from byte 256, the tile sums in 16
+// bytes per kSmallSegd lengths.
 int64_t segd_build_scratch_bytes(int64_t n, int64_t m) {
     SegdLayout L(n, m);
     const int64_t ta = (m + kSmallSegd - 1) / kSmallSegd, tb = (L.words + kSmallSegd - 1) / kSmallSegd;
@@ -494,6 +510,7 @@ void segd_build(void *sd, const void *lens_in, int64_t n, int64_t m, void *scrat
     }
     const int64_t tiles = (m + kTile - 1) / kTile;
     const int64_t chunks = L.words > 0 ? (L.words + kChunkWords - 1) / kChunkWords : 1;
+    int *count = (int *)scratch;
     uint64_t *parts = (uint64_t *)((char *)scratch + 256);
     if (tiles > 1) {
         k_segd_sums<<<(unsigned)tiles, kTileThreads, 0, g_stream>>>((const int *)lens_in, m, parts, hdr);
@@ -506,10 +523,10 @@ void segd_build(void *sd, const void *lens_in, int64_t n, int64_t m, void *scrat
     }
     // (at least one tile, so that the header of a descriptor without segments is written)
     k_segd_offsets<<<(unsigned)(tiles > 0 ? tiles : 1), kTileThreads, 0, g_stream>>>(
-        (const int *)lens_in, hdr, lens, offs, nz, wcnt, parts, scanned, n, m);
+        (const int *)lens_in, hdr, lens, offs, nz, wcnt, parts, scanned, count, n, m);
     LAUNCHCHECK();
-    k_segd_words<<<(unsigned)(chunks + (pick ? 1 : 0)), kChunkThreads, 0, g_stream>>>(offs, nz, wcnt, heads, L.words, chunks,
-                                                                                  hdr, n, m, pick);
+    k_segd_words<<<(unsigned)(chunks + (pick ? 1 : 0)), kChunkThreads, 0, g_stream>>>(offs, nz, count, wcnt, heads, L.words,
+                                                                                  chunks, hdr, n, m, pick);
     LAUNCHCHECK();
 }
 

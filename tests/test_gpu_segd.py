@@ -148,3 +148,36 @@ def test_long_vectors_keep_the_widest_tiles(cv, n):
     print("picks", n, picks, flush=True)
     if n >= 1 << 25 and cv.lib.cvlhip_sched_has_model():
         assert picks == [0, 0, 0, 0]
+
+
+# Lengths that do not sum to n: the bitmap holds the heads below n, and every
+# head count is defined (the memory holds garbage before), in both builds.
+def off_sums():
+    rng = np.random.default_rng(17)
+    few = np.array([0, 60, 0, 40], np.int32)
+    many = rng.integers(0, 40, 9000).astype(np.int32)
+    return [("small_short", few, 100_000), ("small_long", many[:4000], 30_000), ("few_short", few, 500_000),
+            ("none", np.zeros(3, np.int32), 400_000), ("many_short", many, 1_000_003), ("chunks_short", many, 1 << 20),
+            ("many_long", many, 100_000), ("chunks_long", many, 1 << 17), ("one_past", few, 8192 * 40 + 1)]
+
+
+@pytest.mark.parametrize("name,lens,n", off_sums(), ids=[s[0] for s in off_sums()])
+def test_lengths_that_do_not_sum_to_n(cv, name, lens, n):
+    import torch
+    print("segd off sum", name, lens.size, n, int(lens.sum()), flush=True)
+    L, m = cv.lib, lens.size
+    buf = torch.full((L.siz_fos(n, m) * 2 + 64,), 0x7F7F7F7F, dtype=torch.int32, device=cv.device)
+    L.mke_fov(buf, torch.from_numpy(lens).to(cv.device), n, m, cv.scratch(L.mke_fov_scratch(n, m)))
+    offs = np.concatenate([[0], np.cumsum(lens.astype(np.int64))])
+    at = offs[:-1][lens > 0]
+    W, o_lens, o_offs, o_nz, o_wcnt, o_heads = layout(n, m)
+    bits = np.zeros((W + 8) * 32, np.uint8)
+    bits[at[at < n]] = 1
+    raw = host(buf).view(np.uint8)
+    i32 = lambda off, k: raw[off:off + 4 * k].view(np.int32)
+    assert list(raw[:16].view(np.int64)) == [n, m]
+    assert np.array_equal(i32(o_offs, m + 1), offs)
+    assert np.array_equal(i32(o_nz, at.size), np.nonzero(lens > 0)[0])
+    assert np.array_equal(raw[o_heads:o_heads + 4 * (W + 8)].view(np.uint32),
+                          np.packbits(bits, bitorder="little").view(np.uint32))
+    assert np.array_equal(i32(o_wcnt, W + 1), np.concatenate([[0], np.cumsum(bits[:W * 32].reshape(W, 32).sum(1, dtype=np.int64))]))

@@ -313,9 +313,10 @@ unsigned long long mailbox_wait(unsigned long long seq);   // host: the value po
 // Where the blocks of a reduction that the host waits for leave their
 // partials: counters that return to 0 with each call, and for each of up to
 // kReducePartials blocks one word per 32 bits of its partial, under the low
-// half of the call's sequence number.  The library's own memory, so that a
-// word carries a number only if that call wrote it; calls that wait for the
-// host never overlap.  Cleared whenever the low half wraps (mailbox_next).
+// half of the call's sequence number.  The library's own memory, one on each
+// device, so that a word carries a number only if that call wrote it; calls
+// that wait for the host never overlap.  Cleared whenever the low half has
+// wrapped since the device's last call.
 constexpr int kReducePartials = 2048;
 constexpr int kShareGroups = 32;
 struct ReduceShare {
@@ -324,7 +325,9 @@ struct ReduceShare {
     } count[1 + kShareGroups];
     uint64_t words[2 * kReducePartials];
 };
-ReduceShare *reduce_share();                            // device address (allocated with the mailbox)
+// The current device's, for the call that posts under seq (allocated on the
+// first); null if it cannot be had.
+ReduceShare *reduce_share(unsigned long long seq);
 
 __device__ __forceinline__ void mailbox_post(Mailbox *mb, unsigned long long seq, unsigned long long bits) {
     __hip_atomic_store(&mb->value, bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);

@@ -75,7 +75,11 @@ __global__ void k_fill_u32(uint32_t *__restrict__ p, uint32_t v, int64_t count) 
 static Mailbox *g_mb_host = nullptr;
 static Mailbox *g_mb_dev = nullptr;
 static unsigned long long g_mb_seq = 0;
-static ReduceShare *g_share = nullptr;
+constexpr int kShareDevices = 64;
+static struct {
+    ReduceShare *at;
+    uint32_t era;                   // high half of the last call's sequence number
+} g_share[kShareDevices];
 
 Mailbox *mailbox_device() {
     if (!g_mb_host) {
@@ -84,20 +88,32 @@ Mailbox *mailbox_device() {
         g_mb_host->seq = 0;
         g_mb_host->value = 0;
         HIPCHECK(hipHostGetDevicePointer((void **)&g_mb_dev, g_mb_host, 0));
-        // synchronous clear, before any kernel can read it
-        HIPCHECK(hipMalloc((void **)&g_share, sizeof(ReduceShare)));
-        HIPCHECK(hipMemset(g_share, 0, sizeof(ReduceShare)));
     }
     return g_mb_dev;
 }
 
-ReduceShare *reduce_share() { return g_share; }
+ReduceShare *reduce_share(unsigned long long seq) {
+    int dev = -1;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kShareDevices) return nullptr;
+    auto &s = g_share[dev];
+    if (!s.at) {
+        void *p = nullptr;
+        const hipError_t e = hipMalloc(&p, sizeof(ReduceShare));
+        if (e != hipSuccess) {
+            (void)hipGetLastError();        // the caller does without
+            return nullptr;
+        }
+        HIPCHECK(hipMemset(p, 0, sizeof(ReduceShare)));      // synchronous: before any kernel reads it
+        s.at = (ReduceShare *)p;
+    } else if (s.era != (uint32_t)(seq >> 32)) {             // the words' numbers wrapped: forget the old ones
+        fill_u32(s.at, 0, sizeof(ReduceShare) / 4);
+    }
+    s.era = (uint32_t)(seq >> 32);
+    return s.at;
+}
 
 unsigned long long mailbox_next() {
-    if ((uint32_t)++g_mb_seq == 0) {       // the words' numbers wrap: forget the old ones
-        ++g_mb_seq;
-        if (g_share) fill_u32(g_share, 0, sizeof(ReduceShare) / 4);
-    }
+    if ((uint32_t)++g_mb_seq == 0) ++g_mb_seq;      // no call's number is 0 in the low half
     return g_mb_seq;
 }
 

@@ -39,10 +39,12 @@ namespace cvlhip {
 // 10^6 17.4 -> 12.9.  (With one counter for all blocks 10^6 ints took 20.5.)
 
 // Result of a reduction: fold the g block partials in block order, then
-// the CVL identity (as the serial loop starts from it), and store it.
+// the CVL identity (as the serial loop starts from it), store it and, with a
+// mailbox (a host's call that has no share), post it.
 template <class Op>
 __global__ __launch_bounds__(kWave) void k_reduce_finish(const typename Op::T *__restrict__ partials, int g,
-                                                         typename Op::T *__restrict__ result) {
+                                                         typename Op::T *__restrict__ result, Mailbox *mb,
+                                                         unsigned long long seq) {
     using T = typename Op::T;
     const Op op;
     const int lane = threadIdx.x;
@@ -60,7 +62,11 @@ __global__ __launch_bounds__(kWave) void k_reduce_finish(const typename Op::T *_
 #pragma unroll
     for (int k = 0; k < K; k++)
         if (k * kWave < g) tot = op(tot, wave_reduce(v[k], op));
-    if (lane == 0) result[0] = op(Op::cvl_id(), tot);
+    if (lane == 0) {
+        const T r = op(Op::cvl_id(), tot);
+        result[0] = r;
+        if (mb) mailbox_post(mb, seq, scalar_bits(r));
+    }
 }
 
 // The result of a reduction of several blocks that the host waits for.  Every
@@ -423,14 +429,15 @@ void reduce_unseg_dev(void *result_dev, const void *s, int64_t n, void *scratch,
         LAUNCHCHECK();
         return;
     }
-    ReduceShare *share = mb ? reduce_share() : nullptr;
     unsigned *err = device_error_word();
+    ReduceShare *share = nullptr;
     int grid;
     if constexpr (!ordered<Op>::value) {
         using S1 = ScanShape<Op, 1>;
         constexpr int64_t step = (int64_t)S1::WAVES * S1::ROW * CVLHIP_REDUCE_U;   // elements per block per step
         const int64_t want = (n + step - 1) / step;
         grid = (int)(want < CVLHIP_REDUCE_GRID ? want : CVLHIP_REDUCE_GRID);
+        if (mb && grid > 1) share = reduce_share(seq);
         k_reduce_strided<Op, CVLHIP_REDUCE_U><<<grid, kBlock, 0, g_stream>>>(
             (const T *)s, n, partials, (T *)result_dev, al16(s), share, mb, seq, err);
     } else {
@@ -439,12 +446,13 @@ void reduce_unseg_dev(void *result_dev, const void *s, int64_t n, void *scratch,
         int64_t per_block = (n + grid - 1) / grid;
         per_block = (per_block + S::WAVES * S::ROW - 1) / (S::WAVES * S::ROW) * (S::WAVES * S::ROW);
         grid = (int)((n + per_block - 1) / per_block);
+        if (mb && grid > 1) share = reduce_share(seq);
         k_reduce<Op, kScanRows><<<grid, kBlock, 0, g_stream>>>((const T *)s, n, per_block, partials,
                                                                (T *)result_dev, al16(s), share, mb, seq, err);
     }
     LAUNCHCHECK();
     if (grid > 1 && !share) {
-        k_reduce_finish<Op><<<1, kWave, 0, g_stream>>>(partials, grid, (T *)result_dev);
+        k_reduce_finish<Op><<<1, kWave, 0, g_stream>>>(partials, grid, (T *)result_dev, mb, seq);
         LAUNCHCHECK();
     }
 }

@@ -511,9 +511,14 @@ __global__ __launch_bounds__(kPartThreads) void k_block_scatter(IndexSource src,
 // 8192).  us against the partition: ints 9000 29 -> 9, 250000 22 -> 8, 10^6
 // 26 -> 17, 2 10^6 31.4 -> 29.2, but 4 10^6 57 -> 56 and 8 10^6 90 -> 105;
 // doubles 10^6 30 -> 18, 4 10^6 77 -> 58, 8 10^6 135 -> 110, 16 10^6 269 -> 227.
+// The partition is left what takes two passes or more (its first pass leaves
+// pairs for another), so larger final blocks raise the limit.
 constexpr int kDirectLog4 = 21, kDirectLog8 = 24;
 template <class T>
-constexpr int direct_log() { return sizeof(T) == 4 ? kDirectLog4 : kDirectLog8; }
+constexpr int direct_log() {
+    constexpr int measured = sizeof(T) == 4 ? kDirectLog4 : kDirectLog8, one_pass = blk_log<T>() + 8;
+    return measured > one_pass ? measured : one_pass;
+}
 
 template <class T, int TH, int ITEMS>
 __global__ __launch_bounds__(TH) void k_permute_direct(IndexSource src, const T *__restrict__ in_val,
@@ -523,6 +528,7 @@ __global__ __launch_bounds__(TH) void k_permute_direct(IndexSource src, const T 
     constexpr int BLOG = blk_log<T>();
     constexpr int kBlocks = 1 << (direct_log<T>() - BLOG);
     static_assert(ITEMS % kPartV == 0, "items per thread come in runs of kPartV");
+    static_assert(direct_log<T>() >= BLOG + 8, "longer vectors take two partition passes");
     __shared__ unsigned s_hist[kBlocks];
     const int tid = threadIdx.x;
     const int blocks = (int)((n - 1) >> BLOG) + 1;
@@ -717,7 +723,10 @@ static void partition_later_levels(const PartLayout<T> &L, IndexSource src, void
         pstride = 1;
     }
     const int64_t blocks = ((n - 1) >> blk_log<T>()) + 1;
-    if (L.levels == l0) usage_error("permute: no level after the first");
+    if (L.levels == l0) {
+        usage_error("permute: no level after the first");
+        return;
+    }
     k_block_scatter<T, false, Local16<T>><<<(unsigned)blocks, kPartThreads, 0, g_stream>>>(
         src, L.local[cur], nullptr, (T *)d, n, cnt, err);
     LAUNCHCHECK();

@@ -14,17 +14,18 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 HOOK = C.CFUNCTYPE(None, C.c_char_p, C.c_uint, C.POINTER(C.c_void_p))
 
 
-def run(script: str, tmp_path, timeout: int = 100) -> str:
-    """`script` in a process whose HIP calls are the fake's; its output."""
+def run(script: str, tmp_path, timeout: int = 100, lib: str = "") -> str:
+    """`script` in a process whose HIP calls are the fake's; its output.
+    lib: another library than the built one."""
     from neslgpu_amd import cvl
-    if not os.path.exists(cvl.LIB_PATH):
+    if not os.path.exists(lib or cvl.LIB_PATH):
         pytest.skip("libcvl_hip.so not built (python -m neslgpu_amd.build)")
     if not shutil.which("gcc"):
         pytest.skip("no gcc")
     so = str(tmp_path / "libfakehip.so")
     subprocess.run(["gcc", "-O1", "-shared", "-fPIC", "-o", so, os.path.join(HERE, "fake_hip.c")], check=True)
     r = subprocess.run([sys.executable, "-c", "import sys; from fake_hip import load, word, Post\n" + script],
-                       env=dict(os.environ, FAKE_HIP=so, PYTHONPATH=os.pathsep.join([HERE, os.path.dirname(HERE)])),
+                       env=dict(os.environ, FAKE_HIP=so, CVLHIP_LIBRARY=lib or cvl.LIB_PATH, PYTHONPATH=os.pathsep.join([HERE, os.path.dirname(HERE)])),
                        capture_output=True, text=True, timeout=timeout)
     assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-4000:]
     return r.stdout

@@ -1,0 +1,42 @@
+"""The tuner's sizes of the partition's final blocks, on the CPU: with each
+of them every length about the limit of the direct permute has a path (one
+that leaves pairs for a second partition pass, or none)."""
+import glob
+import os
+import subprocess
+
+import pytest
+
+import fake_hip
+
+SCRIPT = r'''
+launched = []
+fake, lib = load(lambda name, wgs, args: launched.append(name))
+for log in (13, 14, 18, 20, 21, 22, 23, 24, 25, 26):
+    for n in ((1 << log) - 1, 1 << log, (1 << log) + 1):
+        for ty in "zd":
+            launched.clear()
+            getattr(lib, f"smp_pu{ty}")(1 << 44, 1 << 45, 1 << 46, n, 1 << 47)
+            passes = sum("k_partition" in x for x in launched)
+            assert passes != 1, (n, ty, launched)
+            placed = [x for x in launched if "k_permute_direct" in x or "k_block_scatter" in x]
+            assert len(placed) == 1 and ("k_permute_direct" in placed[0]) <= (passes == 0), (n, ty, launched)
+print("ok")
+'''
+
+
+@pytest.mark.parametrize("log4", [12, 13, 14])
+def test_every_length_has_a_path(tmp_path, log4):
+    from neslgpu_amd import build as B, tune as T
+    assert sorted(T.SPACE["CVLHIP_BLK_LOG4"][0]) == [12, 13, 14]
+    lib = ""
+    if log4 != T.key_value("CVLHIP_BLK_LOG4"):
+        objs = {os.path.basename(o): o for o in glob.glob(os.path.join(B.OBJ, "*.hip.o"))}
+        if not os.path.exists(B.HIPCC) or "partition.hip.o" not in objs:
+            pytest.skip("no hipcc, or no objects of a build")
+        objs["partition.hip.o"] = o = str(tmp_path / "partition.o")
+        lib = str(tmp_path / "libcvl_hip.so")
+        subprocess.run([B.HIPCC, *B.FLAGS, *B.extra_flags(), *T.defines("CVLHIP_BLK_LOG4", log4), "-I", B.OBJ, "-c",
+                        os.path.join(B.CSRC, "partition.hip"), "-o", o], check=True, capture_output=True)
+        subprocess.run([B.HIPCC, f"--offload-arch={B.ARCH}", "-shared", "-fPIC", "-o", lib, *objs.values()], check=True)
+    assert fake_hip.run(SCRIPT, tmp_path, lib=lib).startswith("ok")

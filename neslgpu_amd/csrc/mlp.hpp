@@ -38,11 +38,15 @@ __device__ __forceinline__ float sched_feature(int i, int64_t n, int64_t m, cons
 }
 
 // Schedules a descriptor admits whatever the network predicts.  The flat
-// 8-row schedule (0) takes any descriptor.  The others exist for vectors
-// whose 8-row tiles leave CUs idle, and are admitted below 2^kOthersMaxLogN
-// elements only, the largest length the network was trained on (8 rows are
-// the fastest there; at 2^28 ints in geometric(256) segments a network's pick
-// of 2 rows took 0.84 ms against 0.47).  The per-segment ones (3 thread, 4
+// 8-row schedule (0) takes any descriptor.  The others are admitted for
+// reductions up to 2^kOthersMaxLogN elements, the largest length the network
+// was trained on, and for scans below it.  All arms of eleven kinds of lengths
+// (Zipf, geometric, equal, uniform), total ms of 8 rows / the network's pick /
+// the fastest arm: scans of 2^25 0.83 / 0.85 / 0.83 (doubles 1.60 / 1.76 /
+// 1.60), 8 rows the fastest of every kind there and beyond; reductions of 2^25
+// 0.95 / 0.61 / 0.61 (1.11 / 1.00 / 1.00), short segments gaining from 2 rows;
+// but of 2^27 the pick was a wave per segment at twice the time of 8 rows for
+// geometric(256) lengths.  The per-segment ones (3 thread, 4
 // wave, 5 workgroup) give a segment one lane, wave or workgroup: one long
 // segment serialises them and a few segments leave the chip idle, so each
 // is admitted only when the longest segment is below 2^(kArmMaxClass + 1)
@@ -51,8 +55,9 @@ __device__ __forceinline__ float sched_feature(int i, int64_t n, int64_t m, cons
 constexpr int kArmMaxClass[3] = {5, 12, 15};
 constexpr int kArmMinLogM[3] = {14, 11, 9};
 constexpr int kOthersMaxLogN = 25;
-__host__ __device__ inline unsigned sched_admitted(int cmax, int64_t n, int64_t m) {
-    if (n >= ((int64_t)1 << kOthersMaxLogN)) return 1u;
+__host__ __device__ inline unsigned sched_admitted(int cmax, int64_t n, int64_t m, bool reduce) {
+    const int64_t most = (int64_t)1 << kOthersMaxLogN;
+    if (reduce ? n > most : n >= most) return 1u;
     unsigned a = 7u;
     for (int k = 0; k < 3; k++)
         if (cmax <= kArmMaxClass[k] && m >= ((int64_t)1 << kArmMinLogM[k])) a |= 1u << (3 + k);

@@ -84,7 +84,7 @@ __device__ void sched_pick_block(SegdHeader *hdr, int64_t n, int64_t m, const un
     if (w < 4) {
         const bool red = (w >> 1) != 0, dbl = (w & 1) != 0;
         const float f = sched_feature(lane < kF ? lane : 0, n, m, s_h, s_h + kLenClasses, dbl, red);
-        const int a = mlp_pick_wave(s_P, f, sched_admitted(max_len_class(s_h + kLenClasses), n, m));
+        const int a = mlp_pick_wave(s_P, f, sched_admitted(max_len_class(s_h + kLenClasses), n, m, red));
         if (lane == 0) s_pick[w] = (unsigned)a;
     }
     __syncthreads();

@@ -159,17 +159,17 @@ def features(cv, sd, kind: str, ty: str) -> np.ndarray:
 
 # Schedules a descriptor admits (csrc/mlp.hpp sched_admitted): the thread,
 # wave and workgroup arms only below a longest-segment class and above a
-# segment count; all but flat8 only below 2^OTHERS_MAX_LOG_N elements.
+# segment count; all but flat8 only up to 2^OTHERS_MAX_LOG_N elements, in
+# scans below that.
 ARM_MAX_CLASS = {3: 5, 4: 12, 5: 15}
 ARM_MIN_LOG_M = {3: 14, 4: 11, 5: 9}
-
-
 OTHERS_MAX_LOG_N = 25
 
 
 def admitted(feat: np.ndarray) -> np.ndarray:
     """Boolean mask over ARMS for feature vectors (rows of `feat`), from
-    the segment-class fractions and log2(m)/32 the library computes."""
+    the segment-class fractions, log2(n)/32, log2(m)/32 and the reduction flag
+    the library computes (as floats, which tell lengths apart to 1 in 10^5)."""
     feat = np.atleast_2d(feat)
     classes = (feat.shape[1] - 5) // 2
     segs = feat[:, 3 + classes: 3 + 2 * classes]
@@ -179,8 +179,8 @@ def admitted(feat: np.ndarray) -> np.ndarray:
     ok = np.ones((feat.shape[0], len(ARMS)), bool)
     for a in ARM_MAX_CLASS:
         ok[:, a] = (cmax <= ARM_MAX_CLASS[a]) & (logm >= ARM_MIN_LOG_M[a] - 1e-6)
-    # below 2^OTHERS_MAX_LOG_N elements only (log2(n)/32 is feature 0)
-    ok[:, 1:] &= (feat[:, 0].astype(np.float64) * 32.0 < OTHERS_MAX_LOG_N - 1e-5)[:, None]
+    logn = feat[:, 0].astype(np.float64) * 32.0
+    ok[:, 1:] &= np.where(feat[:, -1] != 0, logn < OTHERS_MAX_LOG_N + 1e-5, logn < OTHERS_MAX_LOG_N - 1e-5)[:, None]
     return ok
 
 

@@ -137,17 +137,31 @@ def test_descriptor_edges(cv, name, lens):
     assert cv.lib.cvlhip_check_device_errors() == 0
 
 
-@pytest.mark.parametrize("n", [(1 << 25) - 1, 1 << 25, 1 << 28])
+@pytest.mark.parametrize("n", [(1 << 25) - 1024, 1 << 25, (1 << 25) + 1024, 1 << 28])
 def test_long_vectors_keep_the_widest_tiles(cv, n):
-    """From 2^25 elements on a descriptor's picks are the 8-row schedule."""
-    m = n // 256
+    """Scans from 2^25 elements on, and reductions above, have the 8-row
+    schedule, whatever a network prefers; below, the network's choice."""
+    import torch
+    from neslgpu_amd import dispatch as D
+    from test_gpu_dispatch import forcing_params
+    L, m = cv.lib, n // 256
     lens = np.full(m, 256, np.int32)
     lens[-1] += n - m * 256
-    sd = cv.segd(lens)
-    picks = [cv.lib.cvlhip_segd_pick(sd, red, size) for red in (0, 1) for size in (4, 8)]
-    print("picks", n, picks, flush=True)
-    if n >= 1 << 25 and cv.lib.cvlhip_sched_has_model():
-        assert picks == [0, 0, 0, 0]
+    saved = torch.empty(D.mlp_dims(L)[3], dtype=torch.float32, device=cv.device)
+    L.cvlhip_sched_get_params(saved)
+    had = L.cvlhip_sched_has_model()
+    try:
+        for arm in (1, 2, 4):
+            L.cvlhip_sched_set_params(torch.from_numpy(forcing_params(D.mlp_dims(L), arm)).to(cv.device))
+            sd = cv.segd(lens)
+            picks = [L.cvlhip_segd_pick(sd, red, size) for red in (0, 1) for size in (4, 8)]
+            print("picks", n, arm, picks, flush=True)
+            scan, red = arm if n < 1 << 25 else 0, arm if n <= 1 << 25 else 0
+            assert picks == [scan, scan, red, red]
+            for (k, op, ty), pick in zip(D.KINDS, picks):
+                assert D.admitted(D.features(cv, sd, k, ty))[0, arm] == (pick == arm)
+    finally:
+        L.cvlhip_sched_set_params(saved if had else None)
 
 
 # Lengths that do not sum to n: the bitmap holds the heads below n, and every

@@ -198,11 +198,14 @@ void gather(void *d, const void *s, const void *idx, const void *f, int64_t n_d,
 // Scatter in which several k may aim at one destination; `win` is n_d ints
 // of scratch.  v: the default of destinations nobody aims at (null: they
 // keep their contents).
-// Few sources (below n_d / 32 of 2^22 or more) go by source: 16 10^6 ints
+// Few sources (below n_d / 32 of 2^21 or more) go by source: 16 10^6 ints
 // in place, 0.1% of them aimed at, 14 us against 34 by destination, 6% 56
 // against 64, 11% 73 against 75; in random order, with a default to copy, 31
 // against 54, 103 against 96, 172 against 138.  Short destinations always go
-// by destination, which is a launch less.
+// by destination, which is a launch less: 1% aimed at in random order with a
+// default, 10^6 ints 15.5 by source and 12.8 by destination, 2 10^6 16.1 and
+// 17.3, 3 10^6 17.3 and 22.0 (doubles 15.8 and 14.2, 18.2 and 19.7, 21.8 and
+// 26.2).
 template <class T>
 void scatter_lww(void *d, const void *s, const void *idx, const void *f, const void *v, int64_t n, int64_t n_d,
                  SegBase sb, void *win) {
@@ -213,7 +216,7 @@ void scatter_lww(void *d, const void *s, const void *idx, const void *f, const v
         return;
     }
     if (!win) { usage_error("permute with collisions needs scratch"); return; }
-    const bool few = n_d >= (1 << 22) && n < n_d / 32;
+    const bool few = n_d >= (1 << 21) && n < n_d / 32;
     if (few) {
         if (v) HIPCHECK(hipMemcpyAsync(d, v, (size_t)n_d * sizeof(T), hipMemcpyDeviceToDevice, g_stream));
         k_unclaim<<<pgrid(n), kBlock, 0, g_stream>>>((int *)win, (const int *)idx, (const int *)f, n, n_d, sb);

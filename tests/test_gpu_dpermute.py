@@ -1,7 +1,7 @@
 """Permutes with collisions and defaults (dpe, dfp, fpm) against numpy's
 assignment in element order (the last writer wins): the ends of the place
 kernel's lanes and workgroups (1024 destinations), both sides of the rule for
-few sources (below n_d / 32 of at least 2^22 destinations), repeated indices,
+few sources (below n_d / 32 of at least 2^21 destinations), repeated indices,
 flags, results over their default vector and off 16-byte alignment, and
 indices out of range."""
 import numpy as np
@@ -12,7 +12,8 @@ from gpu_util import eq, host
 pytestmark = pytest.mark.gpu
 
 SHAPES = [(1, 1), (5, 3), (1000, 1023), (3000, 1024), (1000, 1025), (40_000, 30_000), (1 << 17, 1 << 22),
-          ((1 << 17) - 1, 1 << 22), (1, 1 << 22), (900_000, (1 << 20) + 3), (30_000, (1 << 22) - 1), (0, 2000)]
+          ((1 << 17) - 1, 1 << 22), (1, 1 << 22), (900_000, (1 << 20) + 3), (30_000, (1 << 22) - 1), (0, 2000),
+          (1 << 16, 1 << 21), ((1 << 16) - 1, 1 << 21), (1000, (1 << 21) - 1)]
 
 
 @pytest.fixture(scope="module")

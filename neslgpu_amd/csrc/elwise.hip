@@ -224,43 +224,48 @@ __global__ void k_ext_post(const T *p, Mailbox *mb, unsigned long long seq) {
     if (threadIdx.x == 0) mailbox_post(mb, seq, scalar_bits(*p));
 }
 
-// Segmented distribute and index: a lane makes runs of four consecutive
-// elements, which share one bitmap word.  Its head count gives the segment of
-// the first, the head bits after it those of the others; rows of a wave
-// without a head inside any run look one segment up per run.  Bound by the
-// chain of two or three dependent loads, so a lane of a long vector has two
-// runs' lookups in flight, and there are no branches per element (with them
-// the double distribute below took 16.6 us).  MAKE_SEGDES, DIST and INDEX of
-// ints, one element per lane and lookup -> this: 16 10^6 elements in 100 / 10^6
-// / 4 10^6 segments 85 -> 55, 106 -> 73, 161 -> 123 us; 5 10^6 doubles in 300007:
-// the index kernel 13.9 -> 9.5, the distribute 14.0 -> 13.4.  One run per lane
-// is as fast to 2^20 elements and 5% slower at 16 10^6, four up to 3 us slower.
+// Segmented distribute and index: a lane makes runs of 16 bytes, four ints or
+// two doubles, which share one bitmap word.  Its head count gives the segment
+// of the first element, the head bits after it those of the others; rows of a
+// wave without a head inside any run look one segment up per run.  Bound by
+// the chain of two or three dependent loads, so a lane of a long vector has
+// the lookups of eight elements in flight, else of four, and there are no
+// branches per element (with them the double distribute below took 16.6 us).
+// MAKE_SEGDES, DIST and INDEX of ints, one element per lane and lookup -> this:
+// 16 10^6 elements in 100 / 10^6 / 4 10^6 segments 85 -> 55, 106 -> 73, 161 ->
+// 123 us; 5 10^6 elements in 300007: the index kernel 13.9 -> 9.5.  One run of
+// ints per lane is as fast to 2^20 elements and 5% slower at 16 10^6, four up
+// to 3 us slower.  Doubles, one element per lane and lookup / runs of four, whose
+// two stores each leave half of a line / this: 5 10^6 in 300007 segments 13.1 /
+// 11.6 / 11.0 us, 2^25 in 20000 55.5 / 60.6 / 53.7, 2^26 in 2^22 221 / 172 / 156.
+template <int R>
 struct SegRun {
-    int seg[4];            // (a valid segment past the last element, too)
+    int seg[R];            // (a valid segment past the last element, too)
     unsigned turn;         // bit k > 0: a segment starts at element k
     bool split;            // some run of the wave holds more than one segment
 };
-template <int U>
-__device__ __forceinline__ void seg_runs(const SegdView &sv, int64_t t0, bool ne, SegRun (&r)[U]) {
+template <int R, int U>
+__device__ __forceinline__ void seg_runs(const SegdView &sv, int64_t t0, bool ne, SegRun<R> (&r)[U]) {
+    static_assert(32 % R == 0, "a run lies in one bitmap word");
     uint32_t h[U];
     int c[U];
 #pragma unroll
     for (int u = 0; u < U; u++) {
-        const int64_t e = t0 + ((int64_t)u * kBlock + threadIdx.x) * 4;
+        const int64_t e = t0 + ((int64_t)u * kBlock + threadIdx.x) * R;
         const int64_t w = (e < sv.n ? e : sv.n - 1) >> 5;
         h[u] = sv.heads[w];
         c[u] = sv.wcnt[w];
     }
 #pragma unroll
     for (int u = 0; u < U; u++) {
-        const int64_t e = t0 + ((int64_t)u * kBlock + threadIdx.x) * 4;
+        const int64_t e = t0 + ((int64_t)u * kBlock + threadIdx.x) * R;
         const int64_t f = e < sv.n ? e : sv.n - 1;                 // no bit is set past the last element
         const int sh = (int)(f & 31);
-        r[u].turn = e < sv.n ? (h[u] >> sh) & 14u : 0u;
+        r[u].turn = e < sv.n ? (h[u] >> sh) & ((1u << R) - 2u) : 0u;
         r[u].split = ballot(r[u].turn != 0u) != 0;
         int g = c[u] + __popc(h[u] & ((2u << sh) - 1u)) - 1;       // among the non-empty segments
 #pragma unroll
-        for (int k = 0; k < 4; k++) {
+        for (int k = 0; k < R; k++) {
             g += (r[u].turn >> k) & 1u;
             r[u].seg[k] = g;
         }
@@ -270,55 +275,56 @@ __device__ __forceinline__ void seg_runs(const SegdView &sv, int64_t t0, bool ne
     for (int u = 0; u < U; u++) {
         if (r[u].split) {
 #pragma unroll
-            for (int k = 0; k < 4; k++) r[u].seg[k] = sv.nz[r[u].seg[k]];
+            for (int k = 0; k < R; k++) r[u].seg[k] = sv.nz[r[u].seg[k]];
         } else {
             r[u].seg[0] = sv.nz[r[u].seg[0]];
         }
     }
 }
-template <class T>
-__device__ __forceinline__ void store_run(T *d, int64_t e, int64_t n, bool aligned, const T (&x)[4]) {
-    constexpr int V = ew_lane<T>();
-    using VT = typename EwVec<T, V>::type;
-    if (aligned && e + 4 <= n) {
+// A run is one 16-byte store.
+template <class T, int R>
+__device__ __forceinline__ void store_run(T *d, int64_t e, int64_t n, bool aligned, const T (&x)[R]) {
+    static_assert(R == ew_lane<T>(), "16 bytes");
+    using VT = typename EwVec<T, R>::type;
+    if (aligned && e + R <= n) {
+        VT o;
 #pragma unroll
-        for (int q = 0; q < 4 / V; q++) {
-            VT o;
-#pragma unroll
-            for (int k = 0; k < V; k++) o[k] = x[q * V + k];
-            *(VT *)(d + e + q * V) = o;
-        }
+        for (int k = 0; k < R; k++) o[k] = x[k];
+        *(VT *)(d + e) = o;
     } else {
 #pragma unroll
-        for (int k = 0; k < 4; k++)
+        for (int k = 0; k < R; k++)
             if (e + k < n) d[e + k] = x[k];
     }
 }
 
 template <class T, int U>
 __global__ __launch_bounds__(kBlock) void k_dist_seg(T *__restrict__ d, const T *__restrict__ v, SegdView sv, int aligned) {
-    const int64_t t0 = (int64_t)blockIdx.x * (kBlock * 4 * U);
-    SegRun r[U];
+    constexpr int R = ew_lane<T>();
+    const int64_t t0 = (int64_t)blockIdx.x * (kBlock * R * U);
+    SegRun<R> r[U];
     seg_runs(sv, t0, sv.all_nonempty(), r);
-    T x[U][4];
+    T x[U][R];
 #pragma unroll
     for (int u = 0; u < U; u++) {
         if (r[u].split) {
 #pragma unroll
-            for (int k = 0; k < 4; k++) x[u][k] = v[r[u].seg[k]];
+            for (int k = 0; k < R; k++) x[u][k] = v[r[u].seg[k]];
         } else {
-            x[u][0] = x[u][1] = x[u][2] = x[u][3] = v[r[u].seg[0]];
+            const T one = v[r[u].seg[0]];
+#pragma unroll
+            for (int k = 0; k < R; k++) x[u][k] = one;
         }
     }
 #pragma unroll
-    for (int u = 0; u < U; u++) store_run(d, t0 + ((int64_t)u * kBlock + threadIdx.x) * 4, sv.n, aligned, x[u]);
+    for (int u = 0; u < U; u++) store_run(d, t0 + ((int64_t)u * kBlock + threadIdx.x) * R, sv.n, aligned, x[u]);
 }
 
 template <int U>
 __global__ __launch_bounds__(kBlock) void k_index_seg(int *__restrict__ d, const int *__restrict__ init,
                                                       const int *__restrict__ st, SegdView sv, int aligned) {
     const int64_t t0 = (int64_t)blockIdx.x * (kBlock * 4 * U);
-    SegRun r[U];
+    SegRun<4> r[U];
     seg_runs(sv, t0, sv.all_nonempty(), r);
     int x[U][4];
 #pragma unroll
@@ -348,11 +354,11 @@ __global__ __launch_bounds__(kBlock) void k_index_seg(int *__restrict__ d, const
 
 template <class T>
 static void launch_dist_seg(void *d, const void *v, SegdView sv) {
-    constexpr int T1 = kBlock * 4;
+    constexpr int R = ew_lane<T>(), T1 = kBlock * R;
     if (sv.n < kEwLongMin)
-        k_dist_seg<T, 1><<<grid_for(sv.n, T1), kBlock, 0, g_stream>>>((T *)d, (const T *)v, sv, ew_aligned(d));
+        k_dist_seg<T, 4 / R><<<grid_for(sv.n, T1 * (4 / R)), kBlock, 0, g_stream>>>((T *)d, (const T *)v, sv, ew_aligned(d));
     else
-        k_dist_seg<T, 2><<<grid_for(sv.n, T1 * 2), kBlock, 0, g_stream>>>((T *)d, (const T *)v, sv, ew_aligned(d));
+        k_dist_seg<T, 8 / R><<<grid_for(sv.n, T1 * (8 / R)), kBlock, 0, g_stream>>>((T *)d, (const T *)v, sv, ew_aligned(d));
     LAUNCHCHECK();
 }
 

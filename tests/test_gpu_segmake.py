@@ -1,4 +1,4 @@
-"""Segmented distribute and index: runs of four elements per lane, at the
+"""Segmented distribute and index: runs of four ints or two doubles, at the
 ends of tiles (1024 elements; 2048 from 2^21 elements on), segments shorter
 and longer than a run, empty ones first, last and in a row, on aligned and
 unaligned results."""

@@ -157,11 +157,13 @@ __device__ __forceinline__ void or_publish(const uint32_t (&v)[NW], unsigned *__
 // ORW: bits that differ from key 0, two words per tile) folded with the
 // segment words of k_seg_or (when segmented); bit p of the posted mask is
 // set when pass p reorders something (key passes first, then segment
-// passes).  One workgroup.
+// passes).  One workgroup.  It also leaves the mask in *word, for the pass
+// behind it.
 constexpr int kOrPostThreads = 1024;
 __global__ __launch_bounds__(kOrPostThreads) void k_or_post(const uint32_t *__restrict__ parts, int64_t nparts,
                                                            const uint32_t *__restrict__ seg_words, int key_passes,
-                                                           int seg_passes, Mailbox *mb, unsigned long long seq) {
+                                                           int seg_passes, Mailbox *mb, unsigned long long seq,
+                                                           unsigned *__restrict__ word) {
     __shared__ uint32_t s_or[kOrPostThreads / kWave][2];
     const int tid = threadIdx.x, w = tid / kWave, lane = tid % kWave;
     uint32_t v[2] = {0, 0};
@@ -193,6 +195,7 @@ __global__ __launch_bounds__(kOrPostThreads) void k_or_post(const uint32_t *__re
             if ((kdiff >> (8 * p)) & 255u) mask |= 1ull << p;
         for (int q = 0; q < seg_passes; q++)
             if ((sdiff >> (8 * q)) & 255u) mask |= 1ull << (key_passes + q);
+        *word = (unsigned)mask;
         mailbox_post(mb, seq, mask);
     }
 }
@@ -455,6 +458,7 @@ struct PassArgs {
     // adds up what lies before its tile itself; starts is not read.
     unsigned *groups;
     int64_t ngroups;
+    const unsigned *runs;    // pass 0, launched before the host knows: does nothing unless bit 0 is set here
     // The last pass with a direct inverse: rank[index] = position, minus the
     // start of the index's segment when rel is set.
     int *rank;
@@ -645,6 +649,9 @@ __global__ __launch_bounds__(TH) void k_rank_pass(PassArgs a) {
     __shared__ unsigned s_placed;                  // FUSE: pairs staged
     __shared__ unsigned s_tile;
 
+    unsigned go = 1u;
+    if constexpr (GRP)
+        if (a.runs) go = *a.runs;
     const int tid = threadIdx.x;
     const int w = tid / kWave, lane = tid % kWave;
     for (int i = tid; i < W * kRadix; i += TH) (&s_cnt[0][0])[i] = 0;
@@ -741,6 +748,8 @@ __global__ __launch_bounds__(TH) void k_rank_pass(PassArgs a) {
         idx[j] = ix;
     }
 loaded:
+    if constexpr (GRP)
+        if (!(go & 1u)) return;          // (asked behind the loads: 1 us a call less than in front of them)
     if (wb + kWaveSpan <= a.n) multisplit<true>(key, a.shift, lane, kWaveSpan, s_cnt[w], dig, loc);
     else multisplit<false>(key, a.shift, lane, a.n - wb, s_cnt[w], dig, loc);
     __syncthreads();
@@ -1108,7 +1117,7 @@ void rank_run(int *rank, const void *s, int64_t n, bool dbl, bool up, const void
         // inverse's counters and column-scans pass 0's counts (or, with
         // grouped tiles, runs pass 0), covering the host's wait and its next
         // launches.
-        unsigned *words = hist;
+        unsigned *words = hist, *mask_word = (unsigned *)(b + L.counters);
         static_assert(kOrCopies * kOrWords * kOrStride <= 12 * kRadix, "the OR words fit the histogram space");
         if (seg_passes) {
             fill_u32(words, 0, kOrCopies * kOrWords * kOrStride);
@@ -1121,7 +1130,7 @@ void rank_run(int *rank, const void *s, int64_t n, bool dbl, bool up, const void
         else launch_hist<kRankThreads, kRankItems, false, true>(a0, tiles, dbl, tile_ofs, nullptr, or_parts);
         const unsigned long long seq = mailbox_next();
         k_or_post<<<1, kOrPostThreads, 0, g_stream>>>(or_parts, tiles, seg_passes ? words : nullptr, key_passes,
-                                                      seg_passes, mailbox_device(), seq);
+                                                      seg_passes, mailbox_device(), seq, mask_word);
         LAUNCHCHECK();
         // An unsegmented rank whose inverse takes two or more partition
         // passes runs the first of them inside its last pass (kFuse): the
@@ -1129,18 +1138,18 @@ void rank_run(int *rank, const void *s, int64_t n, bool dbl, bool up, const void
         // order is never written and read back.
         if (!segmented && !grouped) inv = partition_invert_begin(n, b + L.invert);
         if (grouped) {
-            // Pass 0 runs whether or not its digit varies (a pass over one
-            // digit keeps the order), so that the device works through the
-            // host's wait.
+            // Pass 0 is launched whether or not its digit varies, so that
+            // the device works through the host's wait, and reads the mask
+            // itself (8 10^6 equal ints: 73 us when it runs all the same, 58
+            // so, 56 with the host asked first).
             PassArgs a = a0;
             a.keys_out = keys[0];
             a.oshift = dbl ? 0 : 8;
             a.idx_out = idxs[0];
             a.kout = kbytes;
+            a.runs = mask_word;
             if (small) launch_grouped<kRankSmallThreads, kRankSmallItems>(a, tiles, dbl, false);
             else launch_grouped<kRankThreads, kRankItems>(a, tiles, dbl, false);
-            cur = 0;
-            kshift = a.oshift;
         } else {
             fill_u32(scan_status, 0, 2 * sw * 14);   // status regions: 12 passes, the inverse's counts, pass 0's
             tile_scan(tile_ofs, tiles, nullptr, scan_status + 13 * sw, true, starts);
@@ -1148,6 +1157,10 @@ void rank_run(int *rank, const void *s, int64_t n, bool dbl, bool up, const void
         }
         const unsigned long long mask = mailbox_wait(seq);
         for (int p = 0; p < total; p++) runs[p] = (mask >> p) & 1u;
+        if (grouped && runs[0]) {
+            cur = 0;
+            kshift = dbl ? 0 : 8;
+        }
     }
     int run[12], nrun = 0;
     bool any = false;

@@ -100,3 +100,31 @@ def test_segmented_rank_rules(cv, n):
         cv.lib.rku_lez(d, s, sd, n, lens.size, cv.scratch(cv.lib.rku_lez_scratch(n, lens.size)))
         eq(host(d), O.rank(x, True, lens), f"segmented rank {kind} {n}")
     assert cv.lib.cvlhip_check_device_errors() == 0
+
+
+@pytest.mark.parametrize("n", [16_385, 40_003, (1 << 19) + 3, (1 << 21) + 5])
+def test_ranks_whose_lowest_digit_is_constant(cv, n):
+    """Pass 0 is launched before the host knows that it has nothing to do:
+    ints that vary in higher digits only or not at all, doubles of whole
+    numbers, plain and segmented, up and down, aligned or not."""
+    import torch
+    rng = np.random.default_rng(n)
+    lens = np.bincount(rng.integers(0, 700, n), minlength=700).astype(np.int32)
+    sd, L = cv.segd(lens), cv.lib
+    keys = {"equal": np.full(n, -9, np.int32), "digit 1": (rng.integers(0, 256, n) << 8).astype(np.int32),
+            "digit 3": (rng.integers(-128, 128, n) << 24).astype(np.int32),
+            "digits 1 to 3": (rng.integers(-2 ** 23, 2 ** 23, n) << 8).astype(np.int32),
+            "whole": rng.integers(-500, 500, n).astype(np.float64), "equal d": np.full(n, 0.1)}
+    for kind, x in keys.items():
+        ty = "d" if x.dtype == np.float64 else "z"
+        print("constant low digit", n, kind, flush=True)
+        for shift in (0, 1):
+            s = torch.empty(n + shift, dtype=torch.float64 if ty == "d" else torch.int32, device=cv.device)[shift:]
+            s.copy_(torch.from_numpy(x))
+            d = torch.empty(n, dtype=torch.int32, device=cv.device)
+            for ud in "ud":
+                getattr(L, f"rk{ud}_lu{ty}")(d, s, n, cv.scratch(getattr(L, f"rk{ud}_lu{ty}_scratch")(n)))
+                eq(host(d), O.rank(x, ud == "u"), f"{kind} {n} {ud}")
+        getattr(L, f"rku_le{ty}")(d, s, sd, n, lens.size, cv.scratch(getattr(L, f"rku_le{ty}_scratch")(n, lens.size)))
+        eq(host(d), O.rank(x, True, lens), f"segmented {kind} {n}")
+    assert L.cvlhip_check_device_errors() == 0

@@ -210,8 +210,8 @@ constexpr int pack_block() { return 1024; }
 // cleared and mid-size vectors reach every CU.  us per PACK (count to the
 // host, then this) against the look-back: ints 40000 20 -> 19, 10^6 23 -> 20, 4
 // 10^6 29 -> 24, 16 10^6 62 -> 56; doubles 10^6 22 -> 20, 8 10^6 50 -> 43, 16
-// 10^6 80 -> 73.  Above, the second reading leaves the caches and each tile
-// adds up more than 4096 counts.
+// 10^6 80 -> 73.  Above, the second reading leaves the caches, and the last
+// tiles add up more than 4096 counts of ints, 8192 of doubles.
 constexpr int64_t kPackCountedMax = (int64_t)1 << 24;
 
 // Packs the n elements of s whose flag is set into d, which holds dlim.

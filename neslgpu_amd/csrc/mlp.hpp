@@ -50,9 +50,13 @@ __device__ __forceinline__ float sched_feature(int i, int64_t n, int64_t m, cons
 // wave, 5 workgroup) give a segment one lane, wave or workgroup: one long
 // segment serialises them and a few segments leave the chip idle, so each
 // is admitted only when the longest segment is below 2^(kArmMaxClass + 1)
-// and there are at least 2^kArmMinLogM segments.  cmax: the highest
-// length class holding a segment (-1: none).  Bit a set: schedule a admitted.
-constexpr int kArmMaxClass[3] = {5, 12, 15};
+// and there are at least 2^kArmMinLogM segments.  (A workgroup takes 50 us for
+// 2^16 elements: with that limit the network's pick for 700000 ints in 3500
+// segments, one of them of 60000, took 52 us against 15 in flat tiles; of 209
+// training workloads none is faster for segments above 2^14.)  cmax: the
+// highest length class holding a segment (-1: none).  Bit a set: schedule a
+// admitted.
+constexpr int kArmMaxClass[3] = {5, 12, 13};
 constexpr int kArmMinLogM[3] = {14, 11, 9};
 constexpr int kOthersMaxLogN = 25;
 __host__ __device__ inline unsigned sched_admitted(int cmax, int64_t n, int64_t m, bool reduce) {

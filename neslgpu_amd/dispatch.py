@@ -161,7 +161,7 @@ def features(cv, sd, kind: str, ty: str) -> np.ndarray:
 # wave and workgroup arms only below a longest-segment class and above a
 # segment count; all but flat8 only up to 2^OTHERS_MAX_LOG_N elements, in
 # scans below that.
-ARM_MAX_CLASS = {3: 5, 4: 12, 5: 15}
+ARM_MAX_CLASS = {3: 5, 4: 12, 5: 13}
 ARM_MIN_LOG_M = {3: 14, 4: 11, 5: 9}
 OTHERS_MAX_LOG_N = 25
 

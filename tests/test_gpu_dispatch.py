@@ -190,6 +190,8 @@ def test_per_segment_arms_need_short_segments_in_numbers(cv):
         "const 100": (np.full(n // 100, 100, np.int32), {4, 5}),
         "const 1000": (np.full(n // 1000, 1000, np.int32), {5}),
         "const 20000": (np.full(n // 20000, 20000, np.int32), set()),
+        "const 100 and one of 16383": (np.append(np.full(9000, 100, np.int32), np.int32(16383)), {5}),
+        "const 100 and one of 16384": (np.append(np.full(9000, 100, np.int32), np.int32(16384)), set()),
     }
     try:
         for arm in (3, 4, 5):

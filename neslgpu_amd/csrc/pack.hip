@@ -188,22 +188,6 @@ __global__ __launch_bounds__(B) void k_pack(const T *__restrict__ s, const int *
     }
 }
 
-constexpr int64_t kPackHeader = 256;
-
-template <class T>
-int64_t pack_scratch_bytes(int64_t n) {
-    int64_t tiles = (n + PackShape<T, kPackRows>::TILE - 1) / PackShape<T, kPackRows>::TILE;
-    return kPackHeader + 8 * tiles + 256;
-}
-
-// Threads per pack workgroup (one tile, one look-back).  Measured on MI355X
-// with 8-row tiles and 256 / 512 / 1024 threads: 2^28 int 0.735 / 0.599 /
-// 0.558 ms, 2^27 double 0.462 / 0.458 / 0.459 (16-row tiles of 256
-// threads: 0.694 and 0.578).  Scratch sizes assume 256 threads, the most
-// tiles.
-template <class T>
-constexpr int pack_block() { return 1024; }
-
 // Vectors of several look-back tiles and at most this length count their
 // flags per tile first and pack in tiles an eighth as large: the flags are
 // read twice, from the caches, but no tile waits for another, nothing is
@@ -213,6 +197,27 @@ constexpr int pack_block() { return 1024; }
 // 10^6 80 -> 73.  Above, the second reading leaves the caches, and the last
 // tiles add up more than 4096 counts of ints, 8192 of doubles.
 constexpr int64_t kPackCountedMax = (int64_t)1 << 24;
+constexpr int kPackCountedRows = 4;
+
+constexpr int64_t kPackHeader = 256;
+
+// The look-back tiles' status words, or the counted tiles' counts.
+template <class T>
+int64_t pack_scratch_bytes(int64_t n) {
+    using S = PackShape<T, kPackRows>;
+    using C = PackShape<T, kPackCountedRows>;
+    const int64_t counted = n < kPackCountedMax ? n : kPackCountedMax;
+    const int64_t status = 8 * ((n + S::TILE - 1) / S::TILE), counts = 4 * ((counted + C::TILE - 1) / C::TILE);
+    return kPackHeader + (counts > status ? counts : status) + 256;
+}
+
+// Threads per pack workgroup (one tile, one look-back).  Measured on MI355X
+// with 8-row tiles and 256 / 512 / 1024 threads: 2^28 int 0.735 / 0.599 /
+// 0.558 ms, 2^27 double 0.462 / 0.458 / 0.459 (16-row tiles of 256
+// threads: 0.694 and 0.578).  Scratch sizes assume 256 threads, the most
+// tiles.
+template <class T>
+constexpr int pack_block() { return 1024; }
 
 // Packs the n elements of s whose flag is set into d, which holds dlim.
 template <class T>
@@ -224,9 +229,8 @@ void pack(void *d, const void *s, const void *f, int64_t n, int64_t dlim, void *
     if (!scratch) usage_error("pack called without scratch");
     int64_t tiles = (n + S::TILE - 1) / S::TILE;
     if (tiles > 1 && n <= kPackCountedMax) {
-        constexpr int R = 4;
+        constexpr int R = kPackCountedRows;
         using C = PackShape<T, R, kBlock>;
-        static_assert(8 * C::TILE >= 4 * PackShape<T, kPackRows>::TILE, "the counts fit the status words' scratch");
         const unsigned g = (unsigned)((n + C::TILE - 1) / C::TILE);
         int *counts = (int *)((char *)scratch + kPackHeader);
         k_pack_count<T, R, kBlock><<<g, kBlock, 0, g_stream>>>((const int *)f, n, counts, ((uintptr_t)f & 15) == 0);

@@ -975,8 +975,8 @@ struct RankScratch {
         // together; grouped tiles have no column scan and keep their group
         // counts there
         groups = scan_status = up(status + row * tiles);
-        int64_t scan_bytes = (kRankPasses + 2) * 8 * tile_scan_status_words(tiles);
-        if (n <= kRankDirectMax) scan_bytes = most(scan_bytes, kRankPasses * row * parts(tiles, kRankGroup));
+        const int64_t ngroups = tiles < kRankGroups * kRankGroup ? parts(tiles, kRankGroup) : kRankGroups;
+        const int64_t scan_bytes = most((kRankPasses + 2) * 8 * tile_scan_status_words(tiles), kRankPasses * row * ngroups);
         // the fused last pass's per-tile child counts; the first pass's
         // per-tile OR words
         status2 = up(scan_status + scan_bytes);

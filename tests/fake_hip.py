@@ -3,6 +3,7 @@
 The fake must come first into a process, so a test runs its script in a
 process of its own, with run(); the script calls load()."""
 import ctypes as C
+import glob
 import os
 import shutil
 import subprocess
@@ -29,6 +30,24 @@ def run(script: str, tmp_path, timeout: int = 100, lib: str = "") -> str:
                        capture_output=True, text=True, timeout=timeout)
     assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-4000:]
     return r.stdout
+
+
+def variant(tmp_path, source: str, key: str, value) -> str:
+    """The library with one of the tuner's values for `source`, linked with
+    the objects of the last build ("": it is the built one's)."""
+    from neslgpu_amd import build as B, tune as T
+    assert T.norm(value) in [T.norm(v) for v in T.SPACE[key][0]]
+    if T.norm(value) == T.norm(T.key_value(key)):
+        return ""
+    objs = {os.path.basename(o): o for o in glob.glob(os.path.join(B.OBJ, "*.hip.o"))}
+    if not os.path.exists(B.HIPCC) or source + ".o" not in objs:
+        pytest.skip("no hipcc, or no objects of a build")
+    objs[source + ".o"] = o = str(tmp_path / "variant.o")
+    lib = str(tmp_path / "libcvl_hip.so")
+    subprocess.run([B.HIPCC, *B.FLAGS, *B.extra_flags(), *T.defines(key, value), "-I", B.OBJ, "-c",
+                    os.path.join(B.CSRC, source), "-o", o], check=True, capture_output=True)
+    subprocess.run([B.HIPCC, f"--offload-arch={B.ARCH}", "-shared", "-fPIC", "-o", lib, *objs.values()], check=True)
+    return lib
 
 
 def load(on_launch):

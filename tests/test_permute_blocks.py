@@ -1,10 +1,6 @@
 """The tuner's sizes of the partition's final blocks, on the CPU: with each
 of them every length about the limit of the direct permute has a path (one
 that leaves pairs for a second partition pass, or none)."""
-import glob
-import os
-import subprocess
-
 import pytest
 
 import fake_hip
@@ -27,16 +23,5 @@ print("ok")
 
 @pytest.mark.parametrize("log4", [12, 13, 14])
 def test_every_length_has_a_path(tmp_path, log4):
-    from neslgpu_amd import build as B, tune as T
-    assert sorted(T.SPACE["CVLHIP_BLK_LOG4"][0]) == [12, 13, 14]
-    lib = ""
-    if log4 != T.key_value("CVLHIP_BLK_LOG4"):
-        objs = {os.path.basename(o): o for o in glob.glob(os.path.join(B.OBJ, "*.hip.o"))}
-        if not os.path.exists(B.HIPCC) or "partition.hip.o" not in objs:
-            pytest.skip("no hipcc, or no objects of a build")
-        objs["partition.hip.o"] = o = str(tmp_path / "partition.o")
-        lib = str(tmp_path / "libcvl_hip.so")
-        subprocess.run([B.HIPCC, *B.FLAGS, *B.extra_flags(), *T.defines("CVLHIP_BLK_LOG4", log4), "-I", B.OBJ, "-c",
-                        os.path.join(B.CSRC, "partition.hip"), "-o", o], check=True, capture_output=True)
-        subprocess.run([B.HIPCC, f"--offload-arch={B.ARCH}", "-shared", "-fPIC", "-o", lib, *objs.values()], check=True)
+    lib = fake_hip.variant(tmp_path, "partition.hip", "CVLHIP_BLK_LOG4", log4)
     assert fake_hip.run(SCRIPT, tmp_path, lib=lib).startswith("ok")
